@@ -28,7 +28,8 @@ HOST_SRC = os.path.join(CSRC, "rf_host.hip")
 # torch's C++ headers (tensor data pointers without a Python call).
 PYHOST_SRC = os.path.join(CSRC, "rf_pyhost.cpp")
 INST_SRC = os.path.join(CSRC, "rf_adam8_inst.hip")
-# One object per (apply, moment SR, exact) instance of the step kernel.
+TILE_SRC = os.path.join(CSRC, "rf_tile_inst.hip")
+# One object per (apply, moment SR, exact) instance of the step kernels.
 VARIANTS = [(a, m, e) for a in (0, 1) for m in (0, 1) for e in (0, 1)]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -58,6 +59,10 @@ def _compile_jobs():
         obj = os.path.join(OBJ_DIR, f"rf_adam8_a{a}_m{m}_e{e}.o")
         defs = [f"-DRFI_APPLY={a}", f"-DRFI_MSR={m}", f"-DRFI_EXACT={e}"]
         jobs.append(([HIPCC, *FLAGS, *inc, *defs, "-c", INST_SRC, "-o", obj], obj))
+    for a, m, e in VARIANTS:
+        obj = os.path.join(OBJ_DIR, f"rf_tile_a{a}_m{m}_e{e}.o")
+        defs = [f"-DRFI_APPLY={a}", f"-DRFI_MSR={m}", f"-DRFI_EXACT={e}"]
+        jobs.append(([HIPCC, *FLAGS, *inc, *defs, "-c", TILE_SRC, "-o", obj], obj))
     return jobs
 
 
@@ -92,6 +97,8 @@ def _sources_of(obj: str) -> list:
     dev = [os.path.join(CSRC, "rf_device.h"), os.path.join(CSRC, "rf_tables.h")]
     if obj.endswith("rf_host.o"):
         return [HOST_SRC, *dev, *inc]
+    if os.path.basename(obj).startswith("rf_tile"):
+        return [TILE_SRC, os.path.join(CSRC, "rf_tile.h"), *dev, *inc]
     if obj.endswith(".o"):
         return [INST_SRC, *dev, *inc]
     return [PYHOST_SRC, *inc, __file__]

@@ -72,7 +72,16 @@ constexpr int64_t EW_UNIT = APPLY ? EW_UNIT_FUSED : CHUNK;
 #define RF_PREFETCH_NEXT 1
 #endif
 
-enum : int32_t { KIND_QFAST = 0, KIND_QGEN = 1, KIND_FALLBACK = 2, KIND_FALLBACK_VEC = 3 };
+enum : int32_t {
+    KIND_QFAST = 0,
+    KIND_QGEN = 1,
+    KIND_FALLBACK = 2,
+    KIND_FALLBACK_VEC = 3,
+    KIND_QTILE = 4,  // rf_tile.h: TILE_SPAN elements of whole blocks, a wave
+    KIND_QWAVE = 5,  // a block below TILE_SPAN, a wave
+    KIND_QTEAM = 6,  // a block of up to four spans, a workgroup
+};
+constexpr int64_t TILE_SPAN = 1024;
 
 struct Seg;
 
@@ -2285,9 +2294,10 @@ __device__ void reject_units(const rf_adam8_leaf* __restrict__ leaves, const Seg
         s = seek_seg(segs, nseg, s, u);
         const Seg sg = segs[s];
         const rf_adam8_leaf& L = leaves[sg.leaf];
-        const int64_t span = (sg.kind == KIND_QFAST || sg.kind == KIND_QGEN) ? (int64_t)L.block_size
-                             : sg.kind == KIND_FALLBACK                    ? EW_UNIT<APPLY>
-                                                                           : CHUNK;
+        const int64_t span = (sg.kind == KIND_FALLBACK_VEC)  ? CHUNK
+                             : (sg.kind == KIND_FALLBACK)    ? EW_UNIT<APPLY>
+                             : (sg.kind == KIND_QTILE)       ? TILE_SPAN
+                                                             : (int64_t)L.block_size;
         const int64_t base = (sg.first + (u - sg.unit_start)) * span;
         const int64_t end = min(base + span, L.size);
         for (int64_t e = base + lane; e < end; e += WAVE) {

@@ -47,6 +47,15 @@ adam_kernel_t rf_pick_adam8_a1_m0_e0(int dtype_combo, bool psr, bool nest);
 adam_kernel_t rf_pick_adam8_a1_m0_e1(int dtype_combo, bool psr, bool nest);
 adam_kernel_t rf_pick_adam8_a1_m1_e0(int dtype_combo, bool psr, bool nest);
 adam_kernel_t rf_pick_adam8_a1_m1_e1(int dtype_combo, bool psr, bool nest);
+// Instances of the tile kernel (rf_tile_inst.hip).
+adam_kernel_t rf_pick_tile_a0_m0_e0(bool bf16, bool psr, bool nest);
+adam_kernel_t rf_pick_tile_a0_m0_e1(bool bf16, bool psr, bool nest);
+adam_kernel_t rf_pick_tile_a0_m1_e0(bool bf16, bool psr, bool nest);
+adam_kernel_t rf_pick_tile_a0_m1_e1(bool bf16, bool psr, bool nest);
+adam_kernel_t rf_pick_tile_a1_m0_e0(bool bf16, bool psr, bool nest);
+adam_kernel_t rf_pick_tile_a1_m0_e1(bool bf16, bool psr, bool nest);
+adam_kernel_t rf_pick_tile_a1_m1_e0(bool bf16, bool psr, bool nest);
+adam_kernel_t rf_pick_tile_a1_m1_e1(bool bf16, bool psr, bool nest);
 }  // namespace rf
 
 // ====================================================== standalone kernels ==
@@ -610,6 +619,10 @@ struct StepShape {
 };
 constexpr StepShape STEP_SHAPE_STREAM = {2, 8};
 constexpr StepShape STEP_SHAPE_HEAVY = {4, 16};
+// The tile kernel's units are half as long: the streaming shape in elements.
+// A 202 M-parameter bf16 layer in blocks of 256, runs of 2 and 16 or 32
+// units per wave 437 us, runs of 4 and 16 443 us.
+constexpr StepShape STEP_SHAPE_TILE = {2, 16};
 // Launches of at least this many fast blocks per CU (64 per resident wave
 // at 3 waves per SIMD: far more output than the caches hold) store f32
 // updates and params nontemporally (KHp.upd_nt).
@@ -1207,7 +1220,10 @@ static __device__ __align__(256) uint4 search_tables[SEARCH_BYTES / 16];
 // needs to start at zero (each kernel writes every slot it later reads).
 // Calls that overlap on one GPU (different streams, or threads racing to
 // enqueue) race on it.
-static __device__ __align__(256) uint8_t scratch[RF_NOALLOC_SCRATCH_BYTES];
+// The slack beyond the documented size holds the tile list's sentinel, which
+// the size a tree is checked against leaves out.
+constexpr size_t SCRATCH_SLACK = 256;
+static __device__ __align__(256) uint8_t scratch[RF_NOALLOC_SCRATCH_BYTES + SCRATCH_SLACK];
 
 namespace {
 
@@ -1366,10 +1382,27 @@ constexpr int COMBO_F16 = 4;
 constexpr int GEN_LIST = 5;    // the generic kernel's work list
 constexpr int GEN_TAIL = 6;    // build space: its fallback units, appended after its quantized ones
 constexpr int64_t GEN_WAVE_PER_UNIT_MAX_ROUNDS = 8;  // mixed generic lists up to 8 chip-fulls: one unit per wave
+constexpr int TILE_LIST = 7;   // the tile kernel's work list: its wave units ...
+constexpr int TILE_LEAD = 8;   // ... and (build space) its workgroup units, which lead the list
+constexpr int N_LISTS = 9;
 constexpr int VEC_COMBO = -2;  // a generic list of full-chunk fallback units only
+constexpr int TILE_COMBO = -3;       // the tile list (k_adam8_tile)
+constexpr int TILE_BF16_COMBO = -4;  // the same where every leaf has bf16 params and grads
+inline bool is_tile(int combo) { return combo == TILE_COMBO || combo == TILE_BF16_COMBO; }
+// Largest block the tile kernel holds in registers (a span per wave of a workgroup).
+constexpr int64_t TILE_MAX_BS = WAVES_PER_WG * TILE_SPAN;
 
 adam_kernel_t pick_adam_kernel(bool apply, bool msr, bool psr, bool nest, bool exact, int combo)
 {
+    if (combo == TILE_COMBO || combo == TILE_BF16_COMBO) {
+        const bool b = combo == TILE_BF16_COMBO;
+        if (apply) {
+            if (msr) return exact ? rf_pick_tile_a1_m1_e1(b, psr, nest) : rf_pick_tile_a1_m1_e0(b, psr, nest);
+            return exact ? rf_pick_tile_a1_m0_e1(b, psr, nest) : rf_pick_tile_a1_m0_e0(b, psr, nest);
+        }
+        if (msr) return exact ? rf_pick_tile_a0_m1_e1(b, false, nest) : rf_pick_tile_a0_m1_e0(b, false, nest);
+        return exact ? rf_pick_tile_a0_m0_e1(b, false, nest) : rf_pick_tile_a0_m0_e0(b, false, nest);
+    }
     if (combo == VEC_COMBO) msr = false;  // fallback units have no codes to round
     if (apply) {
         if (msr) return exact ? rf_pick_adam8_a1_m1_e1(combo, psr, nest) : rf_pick_adam8_a1_m1_e0(combo, psr, nest);
@@ -1491,7 +1524,7 @@ struct PlanGroup {
     int64_t seg_offset;
     int64_t units;
     bool tables;   // the list holds quantized units (the kernel stages the LDS tables)
-    int64_t lead;  // generic list: leading quantized units, a workgroup each
+    int64_t lead;  // generic and tile lists: leading quantized units, a workgroup each
 };
 
 struct rf_adam8_plan {
@@ -1605,15 +1638,18 @@ struct WorkLists {
     std::vector<Seg> msegs;          // Magma chunk slots (every leaf unquantized), else empty
     int64_t mchunks = -1;
     std::vector<uint8_t> vecs;       // leaf has 16-byte aligned (vectorised) units
-    std::vector<Seg> gsegs[7];       // build space: the lists of each dtype combination, the generic one and its tail
+    std::vector<Seg> gsegs[N_LISTS]; // build space: the lists of each dtype combination, the generic one and its tail, the tile one
+    size_t tile_sentinel = 0;        // records of `segs` that a tree without a tile list would not have had
 };
 
 rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_t apply, WorkLists& w)
 {
     rf_status st = RF_OK;
     std::vector<Seg>* gsegs = w.gsegs;
-    for (int c = 0; c <= GEN_TAIL; ++c) gsegs[c].clear();
-    int64_t gunits[GEN_TAIL + 1] = {0, 0, 0, 0, 0, 0, 0};
+    for (int c = 0; c < N_LISTS; ++c) gsegs[c].clear();
+    int64_t gunits[N_LISTS] = {};
+    int64_t tile_blocks = 0;  // quantized blocks in the tile list
+    bool tile_bf16 = true;    // all of its leaves have bf16 params and grads
     auto add = [&](int32_t leaf, int combo, int32_t kind, int64_t first, int64_t count) {
         if (count <= 0) return;
         Seg sg{};
@@ -1642,6 +1678,21 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
                 const int64_t nfull = L.size / bs;
                 add(i, combo, KIND_QFAST, 0, nfull);
                 add(i, GEN_LIST, KIND_QGEN, nfull, nb - nfull);
+            } else if (vec && bs % 8 == 0 && bs <= TILE_MAX_BS) {
+                // Aligned leaves of other block sizes (and of 2048 with a
+                // dtype mix that has no k_adam8 instance): the tile kernel.
+                // A 202 M-parameter bf16 layer in blocks of 256: 437 us,
+                // 6.63 ms in the generic kernel's workgroup per block.
+                // Blocks that are not a multiple of 8 elements, or beyond
+                // the registers of a workgroup, stay there.
+                tile_blocks += nb;
+                tile_bf16 &= combo == 3;
+                if (bs < TILE_SPAN && (bs & (bs - 1)) == 0)
+                    add(i, TILE_LIST, KIND_QTILE, 0, (nb * bs + TILE_SPAN - 1) / TILE_SPAN);
+                else if (bs <= TILE_SPAN)
+                    add(i, TILE_LIST, KIND_QWAVE, 0, nb);
+                else
+                    add(i, TILE_LEAD, KIND_QTEAM, 0, nb);
             } else {
                 add(i, GEN_LIST, KIND_QGEN, 0, nb);
             }
@@ -1657,7 +1708,7 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
     // The generic list holds the quantized units (the long ones: two passes
     // over a block) first, a workgroup each, then the fallback units, a wave
     // each.
-    if (gunits[GEN_LIST] > INT32_MAX)
+    if (gunits[GEN_LIST] + tile_blocks > INT32_MAX)
         return fail(RF_ERR_UNSUPPORTED, "more than 2^31 - 1 partial or odd-sized quantized blocks in one launch");
     const int64_t gen_lead = gunits[GEN_LIST];
     for (Seg sg : gsegs[GEN_TAIL]) {
@@ -1665,20 +1716,29 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
         gsegs[GEN_LIST].push_back(sg);
     }
     gunits[GEN_LIST] += gunits[GEN_TAIL];
+    // The tile list: its workgroup units first.
+    const int64_t tile_lead = gunits[TILE_LEAD];
+    for (Seg sg : gsegs[TILE_LIST]) {
+        sg.unit_start += tile_lead;
+        gsegs[TILE_LEAD].push_back(sg);
+    }
+    gsegs[TILE_LIST].swap(gsegs[TILE_LEAD]);
+    gunits[TILE_LIST] += tile_lead;
     std::vector<Seg>& segs = w.segs;
     std::vector<PlanGroup>& groups = w.groups;
     segs.clear();
     groups.clear();
     int64_t units = 0;
-    for (int combo = GEN_LIST; combo >= 0; --combo) {
+    w.tile_sentinel = gunits[TILE_LIST] > 0 && gunits[GEN_LIST] > 0 ? 1 : 0;
+    for (int combo : {TILE_LIST, GEN_LIST, 4, 3, 2, 1, 0}) {
         if (gunits[combo] == 0) continue;
         bool quant = combo != GEN_LIST, vec_only = combo == GEN_LIST;
         for (const Seg& sg : gsegs[combo]) {
             quant |= sg.kind == KIND_QGEN;
             vec_only &= sg.kind == KIND_FALLBACK_VEC;
         }
-        const int kc = combo != GEN_LIST ? combo : (vec_only ? VEC_COMBO : -1);
-        const int64_t lead = kc == -1 ? gen_lead : 0;
+        const int kc = combo == TILE_LIST ? (tile_bf16 ? TILE_BF16_COMBO : TILE_COMBO) : combo != GEN_LIST ? combo : (vec_only ? VEC_COMBO : -1);
+        const int64_t lead = kc == -1 ? gen_lead : is_tile(kc) ? tile_lead : 0;
         groups.push_back({kc, (int64_t)segs.size(), gunits[combo], quant, lead});
         Seg sentinel{};
         sentinel.unit_start = gunits[combo];
@@ -1975,11 +2035,14 @@ void find_carrier(const std::vector<PlanGroup>& groups, bool msr, const PlanGrou
 // wave turn, for a kernel of `occ` workgroups per CU.
 int64_t step_grid(const DevState* ds, int occ, const PlanGroup& g, int32_t run, int64_t per_wave)
 {
-    const int64_t runs = (g.units + run - 1) / run;
-    const int64_t wg_needed = (runs + WAVES_PER_WG - 1) / WAVES_PER_WG;
+    // The tile list's leading units count as a unit per wave of the
+    // workgroup that takes each of them.
+    const int64_t units = is_tile(g.combo) ? g.units + g.lead * (WAVES_PER_WG - 1) : g.units;
+    const int64_t runs = (units + run - 1) / run;
+    const int64_t wg_needed = std::max((runs + WAVES_PER_WG - 1) / WAVES_PER_WG, is_tile(g.combo) ? g.lead : 0);
     const int64_t wg_resident = (int64_t)ds->num_cus * occ;
     const int64_t wg_spread =
-        std::min(wg_needed, (g.units + (int64_t)WAVES_PER_WG * per_wave - 1) / ((int64_t)WAVES_PER_WG * per_wave));
+        std::min(wg_needed, (units + (int64_t)WAVES_PER_WG * per_wave - 1) / ((int64_t)WAVES_PER_WG * per_wave));
     int64_t grid = std::max<int64_t>(1, std::max(std::min(wg_needed, wg_resident), wg_spread));
     const int64_t wg_each = g.lead + (g.units - g.lead + WAVES_PER_WG - 1) / WAVES_PER_WG;
     if (g.combo == -1 && wg_each <= GEN_WAVE_PER_UNIT_MAX_ROUNDS * wg_resident) {
@@ -2121,8 +2184,8 @@ rf_status plan_launch(const rf_adam8_plan* plan, const rf_adam8_leaf* d_leaves, 
         // workgroups (the ragged tree's 1,570 workgroups on 768 slots become
         // 1,536, GPT-2-small's 943 become 768).
         const bool streaming = plan->apply && !msr && !psr && !(f & RF_EXACT);
-        const StepShape shape = streaming ? STEP_SHAPE_STREAM : STEP_SHAPE_HEAVY;
-        k.run = g.combo < 0 ? 1 : shape.run;
+        const StepShape shape = is_tile(g.combo) ? STEP_SHAPE_TILE : streaming ? STEP_SHAPE_STREAM : STEP_SHAPE_HEAVY;
+        k.run = g.combo < 0 && !is_tile(g.combo) ? 1 : shape.run;
         // f32 updates (update-only launches) and f32 params are stored on
         // whole cache lines; nontemporally from UPD_NT_MIN_BLOCKS_PER_CU
         // blocks per CU on.  Three store forms on one GPU (old half-line
@@ -2375,7 +2438,9 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     const size_t o_npart = up(o_nsegs + sizeof(Seg) * w.nsegs.size());
     const size_t o_leafsum = up(o_npart + sizeof(double) * (size_t)(prepass ? std::max<int64_t>(w.nunits, 1) : 1));
     const size_t o_clip = up(o_leafsum + sizeof(double) * (size_t)(prepass ? std::max(w.n_nsegs, 1) : 1));
-    const size_t need = o_clip + 4 * sizeof(float);
+    // (without the tile list's own sentinel, which SCRATCH_SLACK holds)
+    const size_t need = o_clip + 4 * sizeof(float) -
+                        (o_nsegs - up(o_segs + sizeof(Seg) * (w.segs.size() - w.tile_sentinel)));
     if (need > (size_t)RF_NOALLOC_SCRATCH_BYTES)
         return fail(RF_ERR_INVALID, "rf_adam8_step_noalloc: this tree needs " + std::to_string(need) +
                                         " bytes of scratch (leaf and group tables, work lists, norm sums); "
