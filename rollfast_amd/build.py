@@ -11,6 +11,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
@@ -116,23 +117,21 @@ def build(verbose: bool = False, jobs: int | None = None, incremental: bool = Fa
     the path of the built ``.so``.  ``incremental``: recompile only the
     objects older than their sources."""
     os.makedirs(OBJ_DIR, exist_ok=True)
-    max_par = jobs or min(len(VARIANTS) + 1, max(1, os.cpu_count() or 1))
-    pending = [_pyhost_job()] + _compile_jobs()
+    max_par = jobs or min(2 * len(VARIANTS) + 1, max(1, os.cpu_count() or 1))
+    # the moment-SR objects compile longest: first, so that none runs alone at the end
+    pending = sorted(_compile_jobs(), key=lambda job: ("_m1_" not in job[1], "tile" in job[1])) + [_pyhost_job()]
     if incremental:
         pending = [(cmd, obj) for cmd, obj in pending
                    if _stale(pyhost_path() if obj.endswith(".tmp") else obj)]
-    running = []
-    failures = []
-    while pending or running:
-        while pending and len(running) < max_par:
-            cmd, obj = pending.pop(0)
-            if verbose:
-                print(" ".join(cmd), flush=True)
-            running.append((subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True), obj))
-        proc, obj = running.pop(0)
-        out, _ = proc.communicate()
-        if proc.returncode != 0:
-            failures.append((obj, out))
+    def compile_one(job):
+        cmd, obj = job
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        return obj, proc.returncode, proc.stdout
+
+    with ThreadPoolExecutor(max_workers=max_par) as pool:
+        failures = [(obj, out) for obj, code, out in pool.map(compile_one, pending) if code != 0]
     if failures:
         for obj, out in failures:
             sys.stderr.write(f"--- {obj}\n{out}\n")

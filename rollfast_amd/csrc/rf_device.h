@@ -2228,6 +2228,12 @@ __device__ __forceinline__ void dispatch_fallback_vec(const UnitCtx& c, const rf
     }
 }
 
+}  // namespace rf
+
+#include "rf_tile.h"
+
+namespace rf {
+
 // ======================================================== step kernels ===
 // The scalars of the leaf's group in a grouped launch (optax.multi_transform):
 // hl is the launch's KHp with the group's learning rate, weight decay, EMA
@@ -2518,7 +2524,7 @@ constexpr int GEN_WAVES_PER_EU = (VEC_ONLY || MSR || PSR || NEST) ? 1 : 4;
 // The generic list's units over workgroups bid = 0 .. nbid - 1 of a launch:
 // the generic kernel's whole grid, or the leading workgroups of a fast
 // launch the list rides along with (k_adam8, KHp.gsegs).  `lds` holds at
-// least TABLE_BYTES; `red` is 8 words of LDS.
+// least TABLE_BYTES (SEARCH_BYTES with moment SR); `red` is 8 words of LDS.
 template <bool APPLY, bool MSR, bool PSR, bool NEST, bool EXACT, bool VEC_ONLY>
 __device__ __forceinline__ void gen_list(const rf_adam8_leaf* __restrict__ leaves, const Seg* __restrict__ segs,
                                          int64_t total_units, const KHp& h, const uint4* __restrict__ tables,
@@ -2529,7 +2535,7 @@ __device__ __forceinline__ void gen_list(const rf_adam8_leaf* __restrict__ leave
     // tables (null: the list has no quantized units).  The others
     // (element-wise units of small leaves) start at once.
     const int64_t nlead = VEC_ONLY ? 0 : segs[0].lead;
-    if (!VEC_ONLY && tables && (int64_t)bid < nlead) stage_tables(lds, tables);
+    if (!VEC_ONLY && tables && (int64_t)bid < nlead) stage_tables<MSR ? SEARCH_BYTES : TABLE_BYTES>(lds, tables);
 
     const int64_t wave = (int64_t)bid * WAVES_PER_WG + uniform_u32(threadIdx.x / WAVE);
     const int64_t nwaves = (int64_t)nbid * WAVES_PER_WG;
@@ -2553,10 +2559,11 @@ __device__ __forceinline__ void gen_list(const rf_adam8_leaf* __restrict__ leave
     c.kmu0 = c.kmu1 = c.knu0 = c.knu1 = c.kp0 = c.kp1 = 0;
     rf_adam8_leaf L;
     KHp hl = h;  // the current leaf's scalars (its group's, in a grouped launch)
-    // The list's leading quantized units (partial and odd-sized blocks, the
-    // long ones), a workgroup each; then the rest a wave each, handed out
+    // The list's leading quantized units (partial and odd-sized blocks, and
+    // the full ones of a short list), a workgroup each; then the rest a wave each, handed out
     // from the last waves down so that the workgroups of the first phase
     // take none when the workgroups cover every unit.
+    TileSlot sl[2];
     for (int64_t q = bid; q < nlead; q += nbid) {
         s = seek_seg(segs, nseg, s, q);
         const Seg sg = segs[s];
@@ -2564,10 +2571,15 @@ __device__ __forceinline__ void gen_list(const rf_adam8_leaf* __restrict__ leave
             cur_leaf = sg.leaf;
             L = leaves[cur_leaf];
             group_hparams(hl, h, L);
+            flr_setup(hl);
             leaf_context<false>(c, L, hl, MSR, PSR);
             if (h.mpart) c.mbase = h.msegs[cur_leaf].unit_start;
         }
-        unit_qgen_wg<APPLY, MSR, PSR, NEST, EXACT>(c, L, sg.first + (q - sg.unit_start), hl, red);
+        const int64_t blk = sg.first + (q - sg.unit_start);
+        if (sg.kind == KIND_QTEAM)
+            unit_tile<DT_ANY, APPLY, MSR, PSR, EXACT, false, 1>(c, L, hl, NEST, true, team_span(L, blk), sl, false,
+                                                                TileSpan{}, red);
+        else unit_qgen_wg<APPLY, MSR, PSR, NEST, EXACT>(c, L, blk, hl, red);
     }
     for (int64_t u = nlead + (nwaves - 1 - wave); u < total_units; u += nwaves) {
         s = seek_seg(segs, nseg, s, u);
@@ -2597,7 +2609,7 @@ void k_adam8_gen(const rf_adam8_leaf* __restrict__ leaves,
                                                   const Seg* __restrict__ segs, int64_t total_units, KHp h,
                                                   const uint4* __restrict__ tables)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[TABLE_BYTES];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[VEC_ONLY ? 16 : MSR ? SEARCH_BYTES : TABLE_BYTES];
     __shared__ uint32_t red[2 * WAVES_PER_WG];  // absmax bits of a workgroup's block, per wave
     gen_list<APPLY, MSR, PSR, NEST, EXACT, VEC_ONLY>(leaves, segs, total_units, h, tables, lds, red, blockIdx.x,
                                                      gridDim.x);

@@ -48,14 +48,14 @@ adam_kernel_t rf_pick_adam8_a1_m0_e1(int dtype_combo, bool psr, bool nest);
 adam_kernel_t rf_pick_adam8_a1_m1_e0(int dtype_combo, bool psr, bool nest);
 adam_kernel_t rf_pick_adam8_a1_m1_e1(int dtype_combo, bool psr, bool nest);
 // Instances of the tile kernel (rf_tile_inst.hip).
-adam_kernel_t rf_pick_tile_a0_m0_e0(bool bf16, bool psr, bool nest);
-adam_kernel_t rf_pick_tile_a0_m0_e1(bool bf16, bool psr, bool nest);
-adam_kernel_t rf_pick_tile_a0_m1_e0(bool bf16, bool psr, bool nest);
-adam_kernel_t rf_pick_tile_a0_m1_e1(bool bf16, bool psr, bool nest);
-adam_kernel_t rf_pick_tile_a1_m0_e0(bool bf16, bool psr, bool nest);
-adam_kernel_t rf_pick_tile_a1_m0_e1(bool bf16, bool psr, bool nest);
-adam_kernel_t rf_pick_tile_a1_m1_e0(bool bf16, bool psr, bool nest);
-adam_kernel_t rf_pick_tile_a1_m1_e1(bool bf16, bool psr, bool nest);
+adam_kernel_t rf_pick_tile_a0_m0_e0(bool bf16, bool psr);
+adam_kernel_t rf_pick_tile_a0_m0_e1(bool bf16, bool psr);
+adam_kernel_t rf_pick_tile_a0_m1_e0(bool bf16, bool psr);
+adam_kernel_t rf_pick_tile_a0_m1_e1(bool bf16, bool psr);
+adam_kernel_t rf_pick_tile_a1_m0_e0(bool bf16, bool psr);
+adam_kernel_t rf_pick_tile_a1_m0_e1(bool bf16, bool psr);
+adam_kernel_t rf_pick_tile_a1_m1_e0(bool bf16, bool psr);
+adam_kernel_t rf_pick_tile_a1_m1_e1(bool bf16, bool psr);
 }  // namespace rf
 
 // ====================================================== standalone kernels ==
@@ -623,6 +623,18 @@ constexpr StepShape STEP_SHAPE_HEAVY = {4, 16};
 // A 202 M-parameter bf16 layer in blocks of 256, runs of 2 and 16 or 32
 // units per wave 437 us, runs of 4 and 16 443 us.
 constexpr StepShape STEP_SHAPE_TILE = {2, 16};
+// Short lists of full 2048-blocks run in the generic list instead of
+// k_adam8, a workgroup per block: one launch for the tree whatever its
+// dtypes, and four waves on a block's memory latencies and random draws
+// where k_adam8 has one.  Up to 6 blocks per CU for nearest rounding of
+// 16-bit params in the hardware direction, 16 otherwise.  One GPU, a step
+// back to back, k_adam8 and generic launch / merged: 98 blocks f32 21.1 /
+// 7.8 us, bf16 14.7 / 7.6, param SR 44.4 / 9.1, all SR 115.5 / 12.2; 1,568
+// blocks 27.9 / 19.5, 16.9 / 16.1, 46.7 / 24.4, 119.8 / 44.4; 3,141 blocks
+// 36.3 / 31.7, 21.5 / 27.5, 48.6 / 41.7, 125.0 / 77.4; 6,248 blocks 58.3 /
+// 54.3, 38.5 / 48.1, 62.8 / 71.1, 142.7 / 129.4.
+constexpr int64_t MERGE_BLOCKS_PER_CU = 6;
+constexpr int64_t MERGE_BLOCKS_PER_CU_HEAVY = 16;
 // Launches of at least this many fast blocks per CU (64 per resident wave
 // at 3 waves per SIMD: far more output than the caches hold) store f32
 // updates and params nontemporally (KHp.upd_nt).
@@ -1296,7 +1308,7 @@ static __device__ __align__(256) uint4 search_tables[SEARCH_BYTES / 16];
 // Calls that overlap on one GPU (different streams, or threads racing to
 // enqueue) race on it.
 // The slack beyond the documented size holds the tile list's sentinel, which
-// the size a tree is checked against leaves out.
+// a tree is not charged for (WorkLists::charged).
 constexpr size_t SCRATCH_SLACK = 256;
 static __device__ __align__(256) uint8_t scratch[RF_NOALLOC_SCRATCH_BYTES + SCRATCH_SLACK];
 
@@ -1459,7 +1471,8 @@ constexpr int GEN_TAIL = 6;    // build space: its fallback units, appended afte
 constexpr int64_t GEN_WAVE_PER_UNIT_MAX_ROUNDS = 8;  // mixed generic lists up to 8 chip-fulls: one unit per wave
 constexpr int TILE_LIST = 7;   // the tile kernel's work list: its wave units ...
 constexpr int TILE_LEAD = 8;   // ... and (build space) its workgroup units, which lead the list
-constexpr int N_LISTS = 9;
+constexpr int MERGED_LIST = 9; // the generic list with a short tree's full 2048-blocks among its leading units
+constexpr int N_LISTS = 10;
 constexpr int VEC_COMBO = -2;  // a generic list of full-chunk fallback units only
 constexpr int TILE_COMBO = -3;       // the tile list (k_adam8_tile)
 constexpr int TILE_BF16_COMBO = -4;  // the same where every leaf has bf16 params and grads
@@ -1472,11 +1485,11 @@ adam_kernel_t pick_adam_kernel(bool apply, bool msr, bool psr, bool nest, bool e
     if (combo == TILE_COMBO || combo == TILE_BF16_COMBO) {
         const bool b = combo == TILE_BF16_COMBO;
         if (apply) {
-            if (msr) return exact ? rf_pick_tile_a1_m1_e1(b, psr, nest) : rf_pick_tile_a1_m1_e0(b, psr, nest);
-            return exact ? rf_pick_tile_a1_m0_e1(b, psr, nest) : rf_pick_tile_a1_m0_e0(b, psr, nest);
+            if (msr) return exact ? rf_pick_tile_a1_m1_e1(b, psr) : rf_pick_tile_a1_m1_e0(b, psr);
+            return exact ? rf_pick_tile_a1_m0_e1(b, psr) : rf_pick_tile_a1_m0_e0(b, psr);
         }
-        if (msr) return exact ? rf_pick_tile_a0_m1_e1(b, false, nest) : rf_pick_tile_a0_m1_e0(b, false, nest);
-        return exact ? rf_pick_tile_a0_m0_e1(b, false, nest) : rf_pick_tile_a0_m0_e0(b, false, nest);
+        if (msr) return exact ? rf_pick_tile_a0_m1_e1(b, false) : rf_pick_tile_a0_m1_e0(b, false);
+        return exact ? rf_pick_tile_a0_m0_e1(b, false) : rf_pick_tile_a0_m0_e0(b, false);
     }
     if (combo == VEC_COMBO) msr = false;  // fallback units have no codes to round
     if (apply) {
@@ -1611,6 +1624,9 @@ struct rf_adam8_plan {
     int64_t total_units = 0;
     int64_t n_segs = 0;
     std::vector<PlanGroup> groups;
+    std::vector<PlanGroup> merged;      // the merged form of a short list (WorkLists::merged), or empty
+    int64_t nfast = 0;
+    bool light = false;                 // light_leaves of its table
     rf_adam8_leaf* d_leaves = nullptr;  // creation-time pointer table
     Seg* d_segs = nullptr;
     // Global-norm clipping (allocated with the plan): one Seg per non-empty
@@ -1706,6 +1722,8 @@ bool leaf_vec_ok(const rf_adam8_leaf& L, int32_t apply)
 struct WorkLists {
     std::vector<Seg> segs;           // every launch's list, each ending in a sentinel
     std::vector<PlanGroup> groups;   // one launch per list
+    std::vector<PlanGroup> merged;   // the launches with the full 2048-blocks in the generic list (short lists only)
+    int64_t nfast = 0;               // full 2048-blocks with a k_adam8 instance
     int64_t units = 0;
     std::vector<Seg> nsegs;          // norm units (NORM_UNIT elements) of the non-empty leaves
     int32_t n_nsegs = 0;
@@ -1714,10 +1732,16 @@ struct WorkLists {
     int64_t mchunks = -1;
     std::vector<uint8_t> vecs;       // leaf has 16-byte aligned (vectorised) units
     std::vector<Seg> gsegs[N_LISTS]; // build space: the lists of each dtype combination, the generic one and its tail, the tile one
-    size_t tile_sentinel = 0;        // records of `segs` that a tree without a tile list would not have had
+    // Records of the lists with every block of another size, and every
+    // generic unit, in one list after the fast ones: what a tree is charged
+    // against rf_adam8_step_noalloc's scratch (`segs` has at most one more).
+    size_t charged = 0;
 };
 
-rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_t apply, WorkLists& w)
+// merge_max: lists of at most this many full 2048-blocks get the merged form
+// too; merged_only: these get no other.
+rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_t apply, int64_t merge_max,
+                           bool merged_only, WorkLists& w)
 {
     rf_status st = RF_OK;
     std::vector<Seg>* gsegs = w.gsegs;
@@ -1752,7 +1776,7 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
             if (bs == FAST_BS && vec && combo >= 0) {
                 const int64_t nfull = L.size / bs;
                 add(i, combo, KIND_QFAST, 0, nfull);
-                add(i, GEN_LIST, KIND_QGEN, nfull, nb - nfull);
+                add(i, GEN_LIST, KIND_QTEAM, nfull, nb - nfull);
             } else if (vec && bs % 8 == 0 && bs <= TILE_MAX_BS) {
                 // Aligned leaves of other block sizes (and of 2048 with a
                 // dtype mix that has no k_adam8 instance): the tile kernel.
@@ -1785,7 +1809,29 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
     // each.
     if (gunits[GEN_LIST] + tile_blocks > INT32_MAX)
         return fail(RF_ERR_UNSUPPORTED, "more than 2^31 - 1 partial or odd-sized quantized blocks in one launch");
+    // A second form of the generic list for short lists of full 2048-blocks:
+    // these as leading units too (MERGE_BLOCKS_PER_CU).
+    int64_t nfast = 0;
+    for (int c = 0; c <= COMBO_F16; ++c) nfast += gunits[c];
     const int64_t gen_lead = gunits[GEN_LIST];
+    w.nfast = nfast;
+    if (nfast > 0 && nfast <= merge_max) {
+        gsegs[MERGED_LIST] = gsegs[GEN_LIST];
+        gunits[MERGED_LIST] = gen_lead;
+        for (int c = 0; c <= COMBO_F16; ++c) {
+            for (Seg sg : gsegs[c]) {
+                sg.unit_start += gunits[MERGED_LIST];
+                sg.kind = KIND_QTEAM;
+                gsegs[MERGED_LIST].push_back(sg);
+            }
+            gunits[MERGED_LIST] += gunits[c];
+        }
+        for (Seg sg : gsegs[GEN_TAIL]) {
+            sg.unit_start += gen_lead + nfast;
+            gsegs[MERGED_LIST].push_back(sg);
+        }
+        gunits[MERGED_LIST] += gunits[GEN_TAIL];
+    }
     for (Seg sg : gsegs[GEN_TAIL]) {
         sg.unit_start += gunits[GEN_LIST];
         gsegs[GEN_LIST].push_back(sg);
@@ -1803,18 +1849,34 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
     std::vector<PlanGroup>& groups = w.groups;
     segs.clear();
     groups.clear();
+    w.merged.clear();
     int64_t units = 0;
-    w.tile_sentinel = gunits[TILE_LIST] > 0 && gunits[GEN_LIST] > 0 ? 1 : 0;
-    for (int combo : {TILE_LIST, GEN_LIST, 4, 3, 2, 1, 0}) {
+    w.charged = gsegs[TILE_LIST].size() + gsegs[GEN_LIST].size();
+    if (w.charged > 0) ++w.charged;
+    for (int c = 0; c <= COMBO_F16; ++c)
+        if (!gsegs[c].empty()) w.charged += gsegs[c].size() + 1;
+    w.charged = std::max<size_t>(w.charged, 1);
+    for (int combo : {TILE_LIST, MERGED_LIST, GEN_LIST, 4, 3, 2, 1, 0}) {
         if (gunits[combo] == 0) continue;
-        bool quant = combo != GEN_LIST, vec_only = combo == GEN_LIST;
+        const bool generic = combo == GEN_LIST || combo == MERGED_LIST;
+        const bool plain = combo != MERGED_LIST;                        // in `groups`
+        const bool in_merged = combo == TILE_LIST || combo == MERGED_LIST;  // in `merged`
+        if (merged_only && gunits[MERGED_LIST] > 0 && !in_merged) continue;
+        bool quant = !generic, vec_only = generic;
         for (const Seg& sg : gsegs[combo]) {
-            quant |= sg.kind == KIND_QGEN;
+            quant |= sg.kind == KIND_QGEN || sg.kind == KIND_QTEAM;
             vec_only &= sg.kind == KIND_FALLBACK_VEC;
         }
-        const int kc = combo == TILE_LIST ? (tile_bf16 ? TILE_BF16_COMBO : TILE_COMBO) : combo != GEN_LIST ? combo : (vec_only ? VEC_COMBO : -1);
-        const int64_t lead = kc == -1 ? gen_lead : is_tile(kc) ? tile_lead : 0;
-        groups.push_back({kc, (int64_t)segs.size(), gunits[combo], quant, lead});
+        const int kc = combo == TILE_LIST ? (tile_bf16 ? TILE_BF16_COMBO : TILE_COMBO)
+                       : !generic         ? combo
+                                          : (vec_only ? VEC_COMBO : -1);
+        const int64_t lead = kc == -1 ? gen_lead + (plain ? 0 : nfast) : is_tile(kc) ? tile_lead : 0;
+        const PlanGroup group = {kc, (int64_t)segs.size(), gunits[combo], quant, lead};
+        if (plain) {
+            groups.push_back(group);
+            units += gunits[combo];
+        }
+        if (in_merged) w.merged.push_back(group);
         Seg sentinel{};
         sentinel.unit_start = gunits[combo];
         sentinel.leaf = -1;
@@ -1822,8 +1884,9 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
         gsegs[combo].push_back(sentinel);
         mark_list(gsegs[combo], (int32_t)lead);
         segs.insert(segs.end(), gsegs[combo].begin(), gsegs[combo].end());
-        units += gunits[combo];
     }
+    if (gunits[MERGED_LIST] == 0) w.merged.clear();
+    if (merged_only && gunits[MERGED_LIST] > 0) units = gunits[MERGED_LIST] + gunits[TILE_LIST];
     if (segs.empty()) {
         Seg sentinel{};
         sentinel.leaf = -1;
@@ -1882,6 +1945,22 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
     w.nunits = nunits;
     w.mchunks = mchunks;
     return RF_OK;
+}
+
+// Leaves whose fast blocks are light in k_adam8: 16-bit params and grads.
+bool light_leaves(const rf_adam8_leaf* leaves, int32_t n)
+{
+    return std::all_of(leaves, leaves + n, [](const rf_adam8_leaf& L) {
+        return L.moment_kind != RF_MOMENT_QUANTIZED || (L.param_dtype != RF_F32 && L.grad_dtype != RF_F32);
+    });
+}
+
+// Full 2048-blocks up to which a step takes the merged lists.
+int64_t merge_max(const DevState* ds, bool light, uint32_t flags, int32_t apply)
+{
+    const bool sr = (flags & RF_MOMENT_SR) || ((flags & RF_PARAM_SR) && apply);
+    return ds->num_cus *
+           (light && apply && !sr && !(flags & RF_EXACT) ? MERGE_BLOCKS_PER_CU : MERGE_BLOCKS_PER_CU_HEAVY);
 }
 
 int64_t step_grid(const DevState* ds, int occ, const PlanGroup& g, int32_t run, int64_t per_wave);
@@ -1950,7 +2029,7 @@ rf_status rf_adam8_plan_create(const rf_adam8_leaf* leaves, int32_t n_leaves, in
     rf_status st = device_state(&ds);
     if (st != RF_OK) return st;
     WorkLists w;
-    st = build_work_lists(leaves, n_leaves, apply, w);
+    st = build_work_lists(leaves, n_leaves, apply, MERGE_BLOCKS_PER_CU_HEAVY * ds->num_cus, false, w);
     if (st != RF_OK) return st;
     std::vector<Seg>& segs = w.segs;
     std::vector<Seg>& nsegs = w.nsegs;
@@ -1969,6 +2048,9 @@ rf_status rf_adam8_plan_create(const rf_adam8_leaf* leaves, int32_t n_leaves, in
     p->total_units = units;
     p->n_segs = (int64_t)segs.size();
     p->groups = w.groups;
+    p->merged = w.merged;
+    p->nfast = w.nfast;
+    p->light = light_leaves(leaves, n_leaves);
     p->cover = bits_cover(leaves, n_leaves);
     p->shape.assign(leaves, leaves + n_leaves);
     p->vec = w.vecs;
@@ -2016,6 +2098,7 @@ rf_status rf_adam8_plan_info(const rf_adam8_plan* plan, int64_t* launches, int64
         const PlanGroup *gen = nullptr, *carrier = nullptr;
         find_carrier(plan->groups, false, &gen, &carrier);
         *launches = (int64_t)plan->groups.size() - (carrier ? 1 : 0);
+        if (!plan->merged.empty()) *launches = std::min(*launches, (int64_t)plan->merged.size());
     }
     if (leaves) *leaves = plan->n_leaves;
     if (units) *units = plan->total_units;
@@ -2237,11 +2320,13 @@ rf_status plan_launch(const rf_adam8_plan* plan, const rf_adam8_leaf* d_leaves, 
     // launch instead of two.
     const PlanGroup* gen = nullptr;
     const PlanGroup* carrier = nullptr;
-    find_carrier(plan->groups, msr, &gen, &carrier);
+    const bool merged = !plan->merged.empty() && plan->nfast <= merge_max(ds, plan->light, f, plan->apply);
+    const std::vector<PlanGroup>& groups = merged ? plan->merged : plan->groups;
+    find_carrier(groups, msr, &gen, &carrier);
     k.gsegs = nullptr;
     k.gunits = 0;
     k.gwgs = 0;
-    for (const PlanGroup& g : plan->groups) {
+    for (const PlanGroup& g : groups) {
         if (carrier && &g == gen) continue;
         adam_kernel_t fn =
             pick_adam_kernel(plan->apply != 0, msr, psr, (f & RF_NESTEROV) != 0, (f & RF_EXACT) != 0, g.combo);
@@ -2494,7 +2579,7 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     std::lock_guard<std::mutex> order(ds->noalloc_mu);
     // Host-side lists in per-thread buffers that keep their capacity.
     thread_local WorkLists w;
-    st = build_work_lists(leaves, n_leaves, apply, w);
+    st = build_work_lists(leaves, n_leaves, apply, merge_max(ds, light_leaves(leaves, n_leaves), hp->flags, apply), true, w);
     if (st != RF_OK) return st;
 
     // Scratch layout: what the host stages (leaf table, group table, step and
@@ -2511,9 +2596,8 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     const size_t o_npart = up(o_nsegs + sizeof(Seg) * w.nsegs.size());
     const size_t o_leafsum = up(o_npart + sizeof(double) * (size_t)(prepass ? std::max<int64_t>(w.nunits, 1) : 1));
     const size_t o_clip = up(o_leafsum + sizeof(double) * (size_t)(prepass ? std::max(w.n_nsegs, 1) : 1));
-    // (without the tile list's own sentinel, which SCRATCH_SLACK holds)
-    const size_t need = o_clip + 4 * sizeof(float) -
-                        (o_nsegs - up(o_segs + sizeof(Seg) * (w.segs.size() - w.tile_sentinel)));
+    // charged with WorkLists::charged records; SCRATCH_SLACK holds one more
+    const size_t need = o_clip + 4 * sizeof(float) - o_nsegs + up(o_segs + sizeof(Seg) * w.charged);
     if (need > (size_t)RF_NOALLOC_SCRATCH_BYTES)
         return fail(RF_ERR_INVALID, "rf_adam8_step_noalloc: this tree needs " + std::to_string(need) +
                                         " bytes of scratch (leaf and group tables, work lists, norm sums); "
@@ -2541,7 +2625,10 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     plan.group_cap = group_cap;
     plan.total_units = w.units;
     plan.n_segs = (int64_t)w.segs.size();
-    plan.groups.swap(w.groups);  // lent for the launch, then handed back with its capacity
+    plan.groups.swap(w.groups);  // lent for the launch, then handed back with their capacity
+    plan.merged.swap(w.merged);
+    plan.nfast = w.nfast;
+    plan.light = light_leaves(leaves, n_leaves);
     plan.d_leaves = (rf_adam8_leaf*)base;
     plan.d_segs = (Seg*)(base + o_segs);
     plan.d_nsegs = (Seg*)(base + o_nsegs);
@@ -2554,6 +2641,7 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     const rf_adam8_group* d_groups = n_groups ? (const rf_adam8_group*)(base + o_groups) : nullptr;
     st = plan_launch(&plan, plan.d_leaves, d_groups, bits_cover(leaves, n_leaves), hp, stream);
     w.groups.swap(plan.groups);
+    w.merged.swap(plan.merged);
     // The next call (any stream) waits for these launches; recorded even
     // after a failed launch, so that whatever was enqueued is covered.
     const hipError_t rec = hipEventRecord(ds->noalloc_ev, (hipStream_t)stream);

@@ -1,8 +1,10 @@
-// rf_tile.h -- the step kernel for quantization blocks of other sizes than
-// 2048 (adam8.py:243-391 takes any block_size; small blocks follow outliers
-// more closely, large ones save scales).
+// rf_tile.h -- the work units of quantization blocks of other sizes than 2048
+// (adam8.py:243-391 takes any block_size; small blocks follow outliers more
+// closely, large ones save scales), for k_adam8_tile (rf_tile_inst.hip), and
+// of 2048-element blocks in lists too short for k_adam8 and leaves' partial
+// last blocks, for the generic list.  Included by rf_device.h.
 //
-// Same execution model as k_adam8 (rf_device.h): a wave owns a span of up to
+// Same execution model as k_adam8: a wave owns a span of up to
 // TILE_SPAN = 1024 consecutive elements, lane l of chunk j the eight from
 // j*512 + 8l, every access a 16-byte (params, grads) or 8-byte (codes) vector
 // access, and the new moments stay in registers until the scales are known,
@@ -15,7 +17,8 @@
 //   KIND_QWAVE  other multiples of 8 below 1024: a wave per block, its last
 //               lanes idle.
 //   KIND_QTEAM  multiples of 8 from 1032 to 4096: a workgroup per block, a
-//               quarter of it per wave, the absmax meeting in LDS.
+//               quarter of it per wave, the absmax meeting in LDS.  In the
+//               generic list: blocks of 2048, one chunk per wave.
 //
 // Partial blocks (a leaf's last) take the same units, the lanes past the
 // leaf's end masked.  The weight-decay mode and eps_root are resolved at run
@@ -34,20 +37,13 @@
 // that); 437 us with the mask-free WHOLE instance.
 #pragma once
 
-#include "rf_device.h"
-
-// Waves per SIMD the tile kernel is register-allocated for.
-#ifndef RF_TILE_WAVES_PER_EU
-#define RF_TILE_WAVES_PER_EU 3
-#endif
-
 namespace rf {
 
 // What a wave works on: code elements [base, base + len) of the leaf.
 struct TileSpan {
     int64_t base;  // a multiple of 8
     int64_t blk0;  // the block of element base
-    int32_t len;   // a multiple of 8, at most TILE_SPAN (0: nothing)
+    int32_t len;   // a multiple of 8, at most J chunks (0: nothing)
     int32_t rem;   // of these, elements of the leaf (the rest is padding)
     int32_t lg;    // log2 of the block size (3 .. 9) where the span holds whole blocks; 10: one block or a part of one
 };
@@ -326,7 +322,21 @@ __device__ __forceinline__ uint2 tile_code8_stream(const UnitCtx& c, const uint3
     return make_uint2(pack4_u8(cc[0], cc[1], cc[2], cc[3]), pack4_u8(cc[4], cc[5], cc[6], cc[7]));
 }
 
-// One span.  TEAM: the workgroup's four waves hold the parts of one block
+// The direction of eight elements, Nesterov's by a uniform branch.
+template <bool EXACT>
+__device__ __forceinline__ void tile_direction8(const KHp& h, bool nest, const float (&m)[8], const float (&v)[8],
+                                                const float (&g)[8], float (&u)[8])
+{
+    if (nest) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) u[t] = adam_direction<true, EXACT>(h, m[t], v[t], g[t]);
+    } else {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) u[t] = adam_direction<false, EXACT>(h, m[t], v[t], g[t]);
+    }
+}
+
+// One span.  `team`: the workgroup's four waves hold the parts of one block
 // (`red`: 8 words of LDS where their absmax bits meet); every wave calls it.
 // `have0`: sl[0] already holds the span's chunk 0; `next`: the wave's next
 // span, of the same leaf, whose chunk 0 is loaded into sl[0] while this one
@@ -334,19 +344,20 @@ __device__ __forceinline__ uint2 tile_code8_stream(const UnitCtx& c, const uint3
 // the leaf, and so is `next`.  That instance has no masks: every path through
 // it issues the same number of memory operations, so the compiler's waits
 // for a chunk's loads leave the later stores in flight.
-template <int32_t DT, bool APPLY, bool MSR, bool PSR, bool NEST, bool EXACT, bool TEAM, bool WHOLE>
-__device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf& L, const KHp& h, const TileSpan& sp,
-                                          TileSlot (&sl)[2], bool have0, const TileSpan& next, uint32_t* red)
+// J: the span's chunks at most.
+template <int32_t DT, bool APPLY, bool MSR, bool PSR, bool EXACT, bool WHOLE, int J>
+__device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf& L, const KHp& h, bool nest, bool team,
+                                          const TileSpan& sp, TileSlot (&sl)[2], bool have0, const TileSpan& next,
+                                          uint32_t* red)
 {
-    constexpr int J = (int)(TILE_SPAN / 512);
     const int lane = threadIdx.x & (WAVE - 1);
     const int32_t pdt = DT == DT_ANY ? L.param_dtype : DT, gdt = DT == DT_ANY ? L.grad_dtype : DT;
     const bool need_p = APPLY || c.wd_mode != WD_OFF;
     // The learning-rate-folded direction (flr_setup) under the same
     // conditions as in k_adam8.
     bool flr = false;
-    if constexpr (APPLY && !NEST && !EXACT)
-        flr = h.flr && h.er2 == 0.0f && pdt == RF_BF16 && (c.wd_mode == WD_BF16 || c.wd_mode == WD_OFF);
+    if constexpr (APPLY && !EXACT)
+        flr = !nest && h.flr && h.er2 == 0.0f && pdt == RF_BF16 && (c.wd_mode == WD_BF16 || c.wd_mode == WD_OFF);
     const float* cbs = (const float*)(c.lds + L_CBS);
     const float* cbu = (const float*)(c.lds + L_CBU);
 
@@ -420,23 +431,22 @@ __device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf&
 #pragma unroll
                 for (int t = 0; t < 8; ++t) {
                     if (__builtin_fmaf(-FLR_CANCEL, fabsf(sum[t]), fabsf(p[t])) > 0.0f)
-                        sum[t] = p[t] + decay_and_scale(h, adam_direction<NEST, true>(h, m[j][t], v[j][t], g[t]), p[t],
+                        sum[t] = p[t] + decay_and_scale(h, adam_direction<false, true>(h, m[j][t], v[j][t], g[t]), p[t],
                                                         c.wd_mode);
                 }
             }
         } else {
-#pragma unroll
-            for (int t = 0; t < 8; ++t) u[t] = adam_direction<NEST, EXACT>(h, m[j][t], v[j][t], g[t]);
+            tile_direction8<EXACT>(h, nest, m[j], v[j], g, u);
             tile_decay8(h, c.wd_mode, u, p);
 #pragma unroll
             for (int t = 0; t < 8; ++t) sum[t] = p[t] + u[t];
             if constexpr (APPLY && !EXACT) {
                 if (cancel_lanes8(sum, u) != 0) {
+                    float ue[8];
+                    tile_direction8<true>(h, nest, m[j], v[j], g, ue);
 #pragma unroll
                     for (int t = 0; t < 8; ++t) {
-                        if (cancels(sum[t], u[t]))
-                            sum[t] = p[t] + decay_and_scale(h, adam_direction<NEST, true>(h, m[j][t], v[j][t], g[t]),
-                                                            p[t], c.wd_mode);
+                        if (cancels(sum[t], u[t])) sum[t] = p[t] + decay_and_scale(h, ue[t], p[t], c.wd_mode);
                     }
                 }
             }
@@ -474,9 +484,14 @@ __device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf&
     // Each block's absmax in all of its lanes.
     const int32_t lg = sp.lg;
     if (lg >= 10) {
-        am[0] = wave_max_u32(max(am[0], am[1]));
-        av[0] = wave_max_u32(max(av[0], av[1]));
-        if constexpr (TEAM) {
+#pragma unroll
+        for (int j = 1; j < J; ++j) {
+            am[0] = max(am[0], am[j]);
+            av[0] = max(av[0], av[j]);
+        }
+        am[0] = wave_max_u32(am[0]);
+        av[0] = wave_max_u32(av[0]);
+        if (!WHOLE && team) {
             const int w = (int)uniform_u32(threadIdx.x / WAVE);
             // (every part that is not empty sees the block's old scales: a part's `odd` makes the block slow in all)
             if (lane == 0) {
@@ -491,8 +506,11 @@ __device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf&
             }
             __syncthreads();  // red is free for the workgroup's next block
         }
-        am[1] = am[0];
-        av[1] = av[0];
+#pragma unroll
+        for (int j = 1; j < J; ++j) {
+            am[j] = am[0];
+            av[j] = av[0];
+        }
     } else {
 #pragma unroll
         for (int j = 0; j < J; ++j) {
@@ -512,12 +530,10 @@ __device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf&
         // A block of the span with a tiny, infinite or NaN scale: the span's
         // blocks are recomputed from their old codes and scales, which are
         // still in place, and coded literally where needed.
-        if constexpr (TEAM) {
-            if (uniform_u32(threadIdx.x / WAVE) == 0) requant_literal<MSR, 1>(c, L, sp.blk0, h);
-        } else {
-            const int64_t nblk = lg >= 10 ? 1 : (int64_t)(sp.len >> lg);
-            for (int64_t b = 0; b < nblk; ++b) requant_literal<MSR, 1>(c, L, sp.blk0 + b, h);
-        }
+        const int64_t nblk = !WHOLE && team ? (uniform_u32(threadIdx.x / WAVE) == 0 ? 1 : 0)
+                             : lg >= 10     ? 1
+                                            : (int64_t)(sp.len >> lg);
+        for (int64_t b = 0; b < nblk; ++b) requant_literal<MSR, 1>(c, L, sp.blk0 + b, h);
         return;
     }
 #pragma unroll
@@ -541,7 +557,7 @@ __device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf&
             st_nt(tile_ptr<uint2>(L.nu, sp.base, 1, eo), wv);
             // Every lane of a block stores its (equal) scales: one store
             // instruction either way, and no branch around it.
-            if (!TEAM || threadIdx.x < WAVE) {
+            if (WHOLE || !team || threadIdx.x < WAVE) {
                 const int64_t blk = sp.blk0 + (eo >> lg);
                 store_scale(L.mu_scales, L.flags, blk, sm[j]);
                 store_scale(L.nu_scales, L.flags, blk, sv[j]);
@@ -562,106 +578,14 @@ __device__ __forceinline__ TileSpan tile_span(const rf_adam8_leaf& L, int64_t lo
     return sp;
 }
 
-// The tile list: its leading KIND_QTEAM units a workgroup each, then a wave
-// per unit in runs of h.run, as in k_adam8.
-template <int32_t DT, bool APPLY, bool MSR, bool PSR, bool NEST, bool EXACT>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(RF_TILE_WAVES_PER_EU))) void k_adam8_tile(
-    const rf_adam8_leaf* __restrict__ leaves, const Seg* __restrict__ segs, int64_t total_units, KHp h,
-    const uint4* __restrict__ tables)
+// The calling wave's part of block blk taken by the workgroup's four waves
+// (KIND_QTEAM): a quarter, rounded up to whole lanes' elements.
+__device__ __forceinline__ TileSpan team_span(const rf_adam8_leaf& L, int64_t blk)
 {
-    constexpr uint32_t LDS_TABLES = MSR ? SEARCH_BYTES : TABLE_BYTES;
-    __shared__ __attribute__((aligned(16))) uint8_t lds[LDS_TABLES];
-    __shared__ uint32_t red[2 * WAVES_PER_WG];
-    stage_tables<LDS_TABLES>(lds, tables);
-    const int64_t wave = (int64_t)blockIdx.x * WAVES_PER_WG + uniform_u32(threadIdx.x / WAVE);
-    const int64_t nwaves = (int64_t)gridDim.x * WAVES_PER_WG;
-    if (gate_rejects(h)) {
-        reject_units<APPLY>(leaves, segs, total_units, wave, nwaves);
-        return;
-    }
-    UnitCtx c;
-    c.lds = lds;
-    c.wtab = nullptr;
-    c.xbuf = nullptr;
-    c.fed = (h.flags & RF_FED_BITS) != 0;
-    c.packed = !c.fed && (h.flags & RF_PACKED_BITS) != 0;
-    c.zero = false;
-    c.mpart = nullptr;
-    c.mbase = 0;
-    clip_context(c, h);
-    c.wd_mode = WD_OFF;
-    c.kmu0 = c.kmu1 = c.knu0 = c.knu1 = c.kp0 = c.kp1 = 0;
-    int32_t s = 0, cur_leaf = -1;
-    const int32_t nseg = segs[0].nseg;
-    const int64_t nlead = segs[0].lead;
-    rf_adam8_leaf L;
-    KHp hl = h;
-    flr_setup(hl);
-    TileSlot sl[2];
-    // Makes unit u's segment current; units in the same segment as the last
-    // one need no load.
-    Seg sg{};
-    int64_t seg_end = -1;
-    auto seek = [&](int64_t u) {
-        if (u < seg_end) return;
-        s = seek_seg(segs, nseg, s, u);
-        sg = segs[s];
-        seg_end = segs[s + 1].unit_start;
-        if (sg.leaf != cur_leaf) {
-            cur_leaf = sg.leaf;
-            L = leaves[cur_leaf];
-            if (h.groups != nullptr) {
-                group_hparams(hl, h, L);
-                flr_setup(hl);
-            }
-            leaf_context<true>(c, L, hl, MSR, PSR);
-        }
-    };
-    for (int64_t q = blockIdx.x; q < nlead; q += gridDim.x) {
-        seek(q);
-        const int64_t blk = sg.first + (q - sg.unit_start);
-        const int64_t bs = L.block_size;
-        // quarters rounded up to whole lanes' elements
-        const int64_t quarter = (bs / 8 + WAVES_PER_WG - 1) / WAVES_PER_WG * 8;
-        const int64_t lo = min(bs, (int64_t)uniform_u32(threadIdx.x / WAVE) * quarter);
-        const int64_t hi = min(bs, lo + quarter);
-        unit_tile<DT, APPLY, MSR, PSR, NEST, EXACT, true, false>(
-            c, L, hl, tile_span(L, blk * bs + lo, blk * bs + hi, blk, 10), sl, false, TileSpan{}, red);
-    }
-    // Wave unit u of the current segment as a span.
-    auto span = [&](int64_t u) {
-        const int64_t idx = sg.first + (u - sg.unit_start);
-        const int64_t bs = L.block_size;
-        if (sg.kind != KIND_QTILE) return tile_span(L, idx * bs, idx * bs + bs, idx, 10);
-        const int32_t lg = 31 - __builtin_clz((uint32_t)bs);
-        const int64_t total = (max((int64_t)1, L.size) + bs - 1) >> lg << lg;
-        return tile_span(L, idx * TILE_SPAN, min(total, idx * TILE_SPAN + TILE_SPAN), idx << (10 - lg), lg);
-    };
-    bool have0 = false;  // sl[0] holds chunk 0 of unit u
-
-    const int64_t units = total_units - nlead;
-    const int64_t run = h.run;
-    const int64_t nruns = (units + run - 1) / run;
-    for (int64_t r = wave; r < nruns; r += nwaves) {
-        const int64_t u_end = min(r * run + run, units);
-        for (int64_t u = r * run; u < u_end; ++u) {
-            seek(nlead + u);
-            const TileSpan sp = span(nlead + u);
-            const bool whole = sp.rem == TILE_SPAN;
-            // a whole next span of the same leaf is prefetched over a whole span
-            const int64_t un = u + 1 < u_end ? u + 1 : (r + nwaves) * run;
-            TileSpan next{};
-            if (whole && un < units && nlead + un < seg_end) {
-                next = span(nlead + un);
-                if (next.rem < TILE_SPAN) next.len = 0;
-            }
-            if (whole)
-                unit_tile<DT, APPLY, MSR, PSR, NEST, EXACT, false, true>(c, L, hl, sp, sl, have0, next, red);
-            else
-                unit_tile<DT, APPLY, MSR, PSR, NEST, EXACT, false, false>(c, L, hl, sp, sl, false, next, red);
-            have0 = next.len > 0;
-        }
-    }
+    const int64_t bs = L.block_size;
+    const int64_t quarter = (bs / 8 + WAVES_PER_WG - 1) / WAVES_PER_WG * 8;
+    const int64_t lo = min(bs, (int64_t)uniform_u32(threadIdx.x / WAVE) * quarter);
+    return tile_span(L, blk * bs + lo, blk * bs + min(bs, lo + quarter), blk, 10);
 }
 
 }  // namespace rf
