@@ -314,4 +314,7 @@ def host_sr_records(quantizer: int) -> np.ndarray:
 def stream_ptr(device=None) -> ctypes.c_void_p:
     import torch
 
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if device is None and raw is not None:  # the handle without a Stream object
+        return ctypes.c_void_p(raw(torch.cuda.current_device()))
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)

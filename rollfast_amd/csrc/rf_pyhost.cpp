@@ -23,6 +23,11 @@
 //   apply_rows(params, updates) -> packed rf_apply_leaf rows and the params
 //       tree for rollfast.apply_updates (see py_apply_rows).
 //
+//   accum_rows(grads, acc) -> packed rf_accum_leaf rows of MultiSteps'
+//       accumulation (see py_accum_rows).
+//
+//   split(k0, k1, n) -> the words of jax.random.split's n keys.
+//
 //   refresh(g, mu, nu, p, rows, table_address, device) -> bool
 //       rows[j] = (i, mref, vref, pref, bufrefs, bufptrs, grad_dtype, size, vec)
 //       Checks that leaf i's moment and param objects are the cached ones
@@ -518,6 +523,116 @@ PyObject* py_apply_rows(PyObject*, PyObject* args)
     return out;
 }
 
+// accum_rows(grads, acc) -> (rows bytes, n rows, device) or None
+//
+// MultiSteps' accumulation over the joint walk of the accumulator and the
+// grads (None: the reset, which has none): contiguous f32 / bf16 / f16
+// tensors on one device, grads of the accumulator's shape whose dtype does
+// not promote the accumulator's.  None / MaskedNode accumulator leaves are
+// left out.  The result None means "not handled here": the Python walk then
+// converts, or raises the error.
+struct AccumWalk {
+    std::string rows;
+    int device = -1;
+    bool reset = false;
+};
+
+int rf_dtype(at::ScalarType t)
+{
+    return t == at::kFloat ? RF_F32 : t == at::kBFloat16 ? RF_BF16 : t == at::kHalf ? RF_F16 : -1;
+}
+
+bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w)
+{
+    if (is_aux(a)) return w.reset || is_grad_leaf(g);
+    if (THPVariable_Check(a)) {
+        const at::Tensor& ta = THPVariable_Unpack(a);
+        rf_accum_leaf row{};
+        row.acc_dtype = rf_dtype(ta.scalar_type());
+        if (row.acc_dtype < 0 || !ta.is_cuda() || !ta.is_contiguous()) return false;
+        if (w.device < 0) w.device = ta.get_device();
+        if (ta.get_device() != w.device) return false;
+        row.acc = ta.data_ptr();
+        row.size = ta.numel();
+        row.grad_dtype = row.acc_dtype;
+        if (!w.reset) {
+            if (!THPVariable_Check(g)) return false;
+            const at::Tensor& tg = THPVariable_Unpack(g);
+            row.grad_dtype = rf_dtype(tg.scalar_type());
+            if (row.grad_dtype < 0 || !tg.is_cuda() || tg.get_device() != w.device || !tg.is_contiguous() ||
+                !tg.sizes().equals(ta.sizes()) || (row.grad_dtype != row.acc_dtype && row.acc_dtype != RF_F32))
+                return false;
+            row.grad = tg.data_ptr();
+        }
+        w.rows.append((const char*)&row, sizeof(row));
+        return true;
+    }
+    if (PyDict_CheckExact(a)) {
+        if (!w.reset && (!PyDict_CheckExact(g) || PyDict_Size(g) != PyDict_Size(a))) return false;
+        PyObject* keys = PyDict_Keys(a);
+        bool ok = keys && PyList_Sort(keys) == 0;
+        for (Py_ssize_t k = 0; ok && k < PyList_GET_SIZE(keys); ++k) {
+            PyObject* key = PyList_GET_ITEM(keys, k);
+            PyObject* ca = PyDict_GetItemWithError(a, key);
+            PyObject* cg = w.reset ? Py_None : PyDict_GetItemWithError(g, key);
+            ok = ca && cg && accum_walk(cg, ca, w);
+        }
+        Py_XDECREF(keys);
+        PyErr_Clear();
+        return ok;
+    }
+    const bool is_list = PyList_CheckExact(a);
+    if (!is_list && !PyTuple_CheckExact(a)) return false;
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(a);
+    if (!w.reset && ((is_list ? !PyList_CheckExact(g) : !PyTuple_CheckExact(g)) || PySequence_Fast_GET_SIZE(g) != n))
+        return false;
+    for (Py_ssize_t k = 0; k < n; ++k)
+        if (!accum_walk(w.reset ? Py_None : PySequence_Fast_GET_ITEM(g, k), PySequence_Fast_GET_ITEM(a, k), w))
+            return false;
+    return true;
+}
+
+PyObject* py_accum_rows(PyObject*, PyObject* args)
+{
+    PyObject *g, *a;
+    if (!PyArg_ParseTuple(args, "OO", &g, &a)) return nullptr;
+    AccumWalk w;
+    w.reset = g == Py_None;
+    if (!accum_walk(g, a, w)) Py_RETURN_NONE;
+    PyObject* rows = PyBytes_FromStringAndSize(w.rows.data(), (Py_ssize_t)w.rows.size());
+    if (!rows) return nullptr;
+    return Py_BuildValue("(Nnn)", rows, (Py_ssize_t)(w.rows.size() / sizeof(rf_accum_leaf)), (Py_ssize_t)w.device);
+}
+
+// split(k0, k1, n) -> tuple of 2n words: threefry2x32(key, (0, i)), i < n, the
+// rounds and key schedule of rollfast_amd/prng.py.
+PyObject* py_split(PyObject*, PyObject* args)
+{
+    unsigned int k0, k1;
+    Py_ssize_t n;
+    if (!PyArg_ParseTuple(args, "IIn", &k0, &k1, &n)) return nullptr;
+    const uint32_t ks[3] = {k0, k1, k0 ^ k1 ^ 0x1BD11BDAu};
+    static const int rot[2][4] = {{13, 15, 26, 6}, {17, 29, 16, 24}};
+    PyObject* out = PyTuple_New(2 * n);
+    for (Py_ssize_t i = 0; out && i < n; ++i) {
+        uint32_t x0 = ks[0], x1 = (uint32_t)i + ks[1];
+        for (uint32_t b = 0; b < 5; ++b) {
+            for (const int r : rot[b & 1]) {
+                x0 += x1;
+                x1 = ((x1 << r) | (x1 >> (32 - r))) ^ x0;
+            }
+            x0 += ks[(b + 1) % 3];
+            x1 += ks[(b + 2) % 3] + b + 1;
+        }
+        PyObject* w0 = PyLong_FromUnsignedLong(x0);
+        PyObject* w1 = PyLong_FromUnsignedLong(x1);
+        PyTuple_SET_ITEM(out, 2 * i, w0);
+        PyTuple_SET_ITEM(out, 2 * i + 1, w1);
+        if (!w0 || !w1) Py_CLEAR(out);
+    }
+    return out;
+}
+
 PyObject* py_set_masked_node_type(PyObject*, PyObject* t)
 {
     if (!PyType_Check(t)) {
@@ -535,6 +650,8 @@ PyMethodDef methods[] = {
     {"refresh", py_refresh, METH_VARARGS, "rewrite the grad pointers of a cached leaf table; False on a mismatch"},
     {"updates_out", py_updates_out, METH_VARARGS, "update-only mode: output buffers and the updates tree"},
     {"apply_rows", py_apply_rows, METH_VARARGS, "apply_updates' leaf table and rebuilt params tree; None if not handled"},
+    {"accum_rows", py_accum_rows, METH_VARARGS, "MultiSteps' accumulation leaf table; None if not handled"},
+    {"split", py_split, METH_VARARGS, "the words of jax.random.split's keys"},
     {"set_masked_node_type", py_set_masked_node_type, METH_O, "the MaskedNode class (a grads leaf)"},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -31,6 +31,7 @@ whose zero multiple is NaN.
 
 from __future__ import annotations
 
+import ctypes
 from typing import Any, Callable, NamedTuple, Optional
 
 import numpy as np
@@ -101,6 +102,17 @@ class _MultiStepsUpdate:
     def _accumulate(self, grads, acc_grads, mode: int, n_acc: int):
         import torch
 
+        # native walk (contiguous tensors in dict / list / tuple containers);
+        # anything else takes the Python walk below, which raises the errors
+        fast = _lib.pyhost().accum_rows(None if mode == _lib.RF_ACC_ZERO else grads, acc_grads)
+        if fast is not None:
+            data, n, device = fast
+            if n:
+                buf = ctypes.create_string_buffer(data, len(data))
+                with torch.cuda.device(device):
+                    _lib.check(_lib.lib().rf_accumulate(ctypes.cast(buf, ctypes.POINTER(_lib.AccumLeaf)), n, int(mode),
+                                                        int(n_acc), _lib.stream_ptr()), "MultiSteps accumulate")
+            return
         a_leaves = _tree.leaves(acc_grads, is_leaf=_is_passthrough_leaf)
         if mode == _lib.RF_ACC_ZERO:
             g_leaves = [None] * len(a_leaves)

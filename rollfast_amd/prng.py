@@ -65,6 +65,23 @@ def _threefry_int(k0: int, k1: int, c0: int, c1: int):
     return x0, x1
 
 
+_native = None  # rf_pyhost's split, or False where the module is not built
+
+
+def _native_split(k0: int, k1: int, num: int):
+    """The words of ``split`` from the native host module (1 us for a step's
+    keys, where the Python integers take 4 us a key); None without it."""
+    global _native
+    if _native is None:
+        try:
+            from . import _lib
+
+            _native = _lib.pyhost().split
+        except (ImportError, OSError, RuntimeError):
+            _native = False
+    return _native(k0, k1, num) if _native else None
+
+
 def as_key(key) -> np.ndarray:
     """Normalise a key (NumPy array, sequence, or host/device tensor) to
     ``uint32[2]``."""
@@ -90,7 +107,10 @@ def split(key, num: int = 2) -> np.ndarray:
     num = int(num)
     if num <= 16:
         k0, k1 = int(k[0]), int(k[1])
-        return np.array([_threefry_int(k0, k1, 0, i) for i in range(num)], dtype=np.uint32).reshape(num, 2)
+        words = _native_split(k0, k1, num)
+        if words is None:
+            words = [_threefry_int(k0, k1, 0, i) for i in range(num)]
+        return np.array(words, dtype=np.uint32).reshape(num, 2)
     i = np.arange(num, dtype=np.uint32)
     y0, y1 = threefry2x32(k, np.zeros_like(i), i)
     return np.stack([y0, y1], axis=1).astype(np.uint32)

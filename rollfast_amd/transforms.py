@@ -114,6 +114,26 @@ def clip_by_global_norm(max_norm: float, *, axis_name=None, partition_axis_names
     return GradientTransformation(init_fn, _ClipUpdate(float(max_norm)))
 
 
+def _first_device(tree):
+    """The device of some leaf of ``tree`` on a ROCm device, or None: the
+    first found, without flattening the tree."""
+    import torch
+
+    if isinstance(tree, torch.Tensor):
+        return tree.device if tree.is_cuda else None
+    if type(tree) is dict:
+        children = tree.values()
+    elif isinstance(tree, (list, tuple)):
+        children = tree
+    else:
+        children = [x for x in _tree.leaves(tree, is_leaf=_is_passthrough_leaf) if isinstance(x, torch.Tensor)]
+    for child in children:
+        device = _first_device(child)
+        if device is not None:
+            return device
+    return None
+
+
 class _ApplyIfFiniteUpdate:
     """``optax.apply_if_finite(inner, max_consecutive_errors).update``.
 
@@ -144,11 +164,7 @@ class _ApplyIfFiniteUpdate:
 
         notfinite_next = safe_int32_increment(int(np.asarray(state.notfinite_count)))
         may_reject = not notfinite_next > self.max_consecutive_errors
-        device = None
-        for leaf in _tree.leaves(updates, is_leaf=_is_passthrough_leaf):
-            if isinstance(leaf, torch.Tensor) and leaf.is_cuda:
-                device = leaf.device
-                break
+        device = _first_device(updates)
         flag = None
         if device is not None:
             if self._flag is None:
