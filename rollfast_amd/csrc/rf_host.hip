@@ -744,32 +744,37 @@ __global__ __launch_bounds__(WG) void k_gnorm_leaf(const Seg* __restrict__ nsegs
 // exactly when all its grads are: squares of finite f32 values (< 2^256)
 // cannot overflow an f64 sum, and an Inf or NaN element makes it Inf or NaN.
 // The leaf sums are added in f32 one after the other (the reference's order):
-// one wave loads 64 of them at a time, the next 64 while every lane adds
-// these from LDS, sixteen broadcast reads in flight ahead of the chain of
-// additions.  2,256 leaves: 167 us when a thread loaded each sum in turn, 27
-// us with a lane read (and its wait states) per sum.
-__global__ void k_gnorm_finish(const double* __restrict__ leafsum, int32_t nseg, float max_norm,
-                               float* __restrict__ clip, float* __restrict__ out, int32_t* __restrict__ finite_out)
+// a workgroup brings up to FINISH_SUMS of them to LDS at once, and its first
+// wave adds them there, sixteen broadcast reads ahead of the chain of
+// additions.  2,256 leaves: 9.2 us; 19.8 when one wave loaded 64 sums at a
+// time (a memory round trip each), 167 when a thread loaded each in turn.
+constexpr int32_t FINISH_SUMS = 4096;
+
+__global__ __launch_bounds__(WG) void k_gnorm_finish(const double* __restrict__ leafsum, int32_t nseg, float max_norm,
+                                                     float* __restrict__ clip, float* __restrict__ out,
+                                                     int32_t* __restrict__ finite_out)
 {
-    __shared__ __attribute__((aligned(16))) float sums[2][WAVE];
-    const int32_t lane = (int32_t)threadIdx.x;  // one workgroup of one wave
+    __shared__ __attribute__((aligned(16))) float sums[FINISH_SUMS];
+    __shared__ int32_t odd[WAVES_PER_WG];
+    const int32_t lane = (int32_t)threadIdx.x;  // one workgroup
     float total = 0.0f;
     bool finite = true;
-    double next = lane < nseg ? leafsum[lane] : 0.0;
-    for (int32_t i0 = 0; i0 < nseg; i0 += WAVE) {
-        const double ls = next;
-        next = i0 + WAVE + lane < nseg ? leafsum[i0 + WAVE + lane] : 0.0;
-        finite = finite && __builtin_isfinite(ls);
-        float* const b = sums[(i0 / WAVE) & 1];
-        b[lane] = (float)ls;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int32_t n = min(WAVE, nseg - i0);
-        if (n == WAVE) {
+    for (int32_t i0 = 0; i0 < nseg; i0 += FINISH_SUMS) {
+        const int32_t n = min(FINISH_SUMS, nseg - i0);
+        if (i0 > 0) __syncthreads();  // the first wave has read the last ones
+#pragma unroll 8
+        for (int32_t i = lane; i < n; i += WG) {
+            const double ls = leafsum[i0 + i];
+            finite = finite && __builtin_isfinite(ls);
+            sums[i] = (float)ls;
+        }
+        __syncthreads();
+        if (lane >= WAVE) continue;
+        const int32_t whole = n / WAVE * WAVE;
+        for (int32_t j = 0; j < whole; j += WAVE) {
             float4 x[WAVE / 4];
 #pragma unroll
-            for (int k = 0; k < WAVE / 4; ++k) x[k] = ((const float4*)b)[k];
+            for (int k = 0; k < WAVE / 4; ++k) x[k] = ((const float4*)(sums + j))[k];
 #pragma unroll
             for (int k = 0; k < WAVE / 4; ++k) {
                 total = total + x[k].x;
@@ -777,12 +782,15 @@ __global__ void k_gnorm_finish(const double* __restrict__ leafsum, int32_t nseg,
                 total = total + x[k].z;
                 total = total + x[k].w;
             }
-        } else {
-            for (int32_t k = 0; k < n; ++k) total = total + b[k];
         }
+        for (int32_t k = whole; k < n; ++k) total = total + sums[k];
     }
-    finite = __builtin_amdgcn_ballot_w64(!finite) == 0;
+    const bool wave_odd = __builtin_amdgcn_ballot_w64(!finite) != 0;
+    if (lane % WAVE == 0) odd[lane / WAVE] = wave_odd ? 1 : 0;
+    __syncthreads();
     if (lane != 0) return;
+#pragma unroll
+    for (int k = 0; k < WAVES_PER_WG; ++k) finite = finite && odd[k] == 0;
     const float norm = sqrtf(total);
     const float q = max_norm / (norm + 1e-6f);
     const float scale = (q < 1.0f || q != q) ? q : 1.0f;  // jnp.minimum(1.0, q): NaN propagates
@@ -2259,7 +2267,7 @@ rf_status plan_launch(const rf_adam8_plan* plan, const rf_adam8_leaf* d_leaves, 
         hipLaunchKernelGGL(k_gnorm_leaf, dim3((unsigned)lw), dim3(WG), 0, (hipStream_t)stream, plan->d_nsegs,
                            plan->n_nsegs, plan->d_npart, plan->d_leafsum);
         HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL(k_gnorm_finish, dim3(1), dim3(WAVE), 0, (hipStream_t)stream, plan->d_leafsum,
+        hipLaunchKernelGGL(k_gnorm_finish, dim3(1), dim3(WG), 0, (hipStream_t)stream, plan->d_leafsum,
                            plan->n_nsegs, max_norm, plan->d_clip, max_norm > 0.0f ? hp->clip_out : nullptr,
                            hp->finite_out);
         HIP_TRY(hipGetLastError());
@@ -2836,7 +2844,7 @@ rf_status rf_clip_by_global_norm(const rf_clip_leaf* leaves, int32_t n_leaves, f
         }
     }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_gnorm_finish, dim3(1), dim3(WAVE), 0, s, d_ls, nseg, max_norm, d_cp, stats, nullptr);
+        hipLaunchKernelGGL(k_gnorm_finish, dim3(1), dim3(WG), 0, s, d_ls, nseg, max_norm, d_cp, stats, nullptr);
         e = hipGetLastError();
     }
     if (e == hipSuccess && maxsize > 0) {

@@ -26,6 +26,7 @@ def _expected(leaves):
     ([16383, 16384, 16385, 40001], 0),
     ([3, 4099, 16384 + 2048, 20480], 1),  # grads at an odd element: the element path
     ([13] * 63, 0), ([5] * 64, 0), ([17] * 65, 0), ([9] * 129, 0),
+    ([9] * 4095, 0), ([9] * 4097, 0),     # the sums one LDS load of the final pass takes
     ([16384 * 1100 + 77], 0),             # more than 1024 units of one leaf
 ])
 def test_norm_edges(dtype, sizes, offset):
