@@ -67,8 +67,87 @@ __device__ __forceinline__ void load8_dt(const void* base, int32_t dtype, int64_
     else load8<float>(base, e0, x);
 }
 
-// Standalone quantize_blocks (adam8.py:113-187): one wave per block.  Fast
-// path: 2048-element aligned blocks held in registers; otherwise two passes.
+// Standalone quantize_blocks (adam8.py:113-187).
+struct QuantArgs {
+    const void* x;
+    uint8_t* values;
+    void* scales;
+    const uint32_t* bits;
+    int64_t size;
+    int64_t nblocks;
+    uint32_t k0, k1;
+    int32_t quantizer, x_dtype, scale_dtype, sr;
+};
+
+// The scale of a block from its absmax bits.
+__device__ __forceinline__ float quant_scale(const QuantArgs& q, uint32_t am)
+{
+    const float amax = __uint_as_float(am);
+    if (q.quantizer == RF_Q_SYMMETRIC_INT8) return amax > 0.0f ? amax / 127.0f : 1.0f;
+    return amax > 0.0f ? amax : 1.0f;
+}
+
+__device__ __forceinline__ bool quant_fast(const QuantArgs& q, uint32_t am, float scale)
+{
+    return !q.sr && q.quantizer != RF_Q_SYMMETRIC_INT8 && block_is_fast(am, scale);
+}
+
+// The code of x, element e of the padded blocks.
+__device__ __forceinline__ uint32_t quant_code(const QuantArgs& q, const uint8_t* lds, float xv, float scale, float rs,
+                                               bool fast, int64_t e)
+{
+    if (q.quantizer == RF_Q_SYMMETRIC_INT8) {
+        // adam8.py:143-164 and _round_scaled :446-458
+        float s = xv / scale;
+        s = s < -127.0f ? -127.0f : (s > 127.0f ? 127.0f : s);
+        float r;
+        if (q.sr) {
+            const uint32_t w = q.bits ? q.bits[e] : jax_bits(q.k0, q.k1, (uint64_t)e);
+            const float lo = floorf(s);
+            r = lo + (uniform_from_bits(w) < (s - lo) ? 1.0f : 0.0f);
+        } else {
+            r = rintf(s);
+        }
+        return (uint32_t)(uint8_t)(int8_t)(r == r ? (int)r : 0);
+    }
+    if (fast) {
+        if (q.quantizer == RF_Q_DYNAMIC_SIGNED) return code_signed_fast(lds, xv, scale, rs);
+        return code_unsigned_fast(lds, xv > 0.0f ? xv : 0.0f, scale, rs);
+    }
+    uint32_t w = 0;
+    if (q.sr) w = q.bits ? q.bits[e] : jax_bits(q.k0, q.k1, (uint64_t)e);
+    const float* cb = (const float*)(lds + (q.quantizer == RF_Q_DYNAMIC_UNSIGNED ? L_CBU : L_CBS));
+    return code_literal(cb, xv, scale, q.sr != 0, w);
+}
+
+// The codes of elements e0 .. e0 + 7; of a fast block in batched phases
+// (normalise, candidate reads, threshold reads), 16 independent LDS reads in
+// flight.
+__device__ __forceinline__ uint2 quant_code8(const QuantArgs& q, const uint8_t* lds, const float (&x)[8], float scale,
+                                             float rs, bool fast, int64_t e0)
+{
+    uint32_t cc[8];
+    if (fast) {
+        const bool sgn = q.quantizer == RF_Q_DYNAMIC_SIGNED;
+        float nv[8], tv[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) nv[t] = div_by_scale(sgn ? x[t] : (x[t] > 0.0f ? x[t] : 0.0f), scale, rs);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) cc[t] = sgn ? cand_signed(lds, nv[t]) : cand_unsigned(lds, nv[t]);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) tv[t] = *(const float*)(lds + (sgn ? L_TS : L_TU) + cc[t] * 4u);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) cc[t] += nv[t] >= tv[t] ? 1u : 0u;
+    } else {
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+            cc[t] = quant_code(q, lds, x[t], scale, rs, false, e0 + t);
+    }
+    return make_uint2(pack4_u8(cc[0], cc[1], cc[2], cc[3]), pack4_u8(cc[4], cc[5], cc[6], cc[7]));
+}
+
+// One wave per block.  Fast path: 2048-element aligned blocks held in
+// registers; otherwise two passes, element by element.
 __global__ __launch_bounds__(WG) void k_quantize(int32_t quantizer, const void* __restrict__ x, int32_t x_dtype,
                                                  int64_t size, int64_t bs, int64_t nblocks, int32_t sr, uint32_t k0,
                                                  uint32_t k1, const uint32_t* __restrict__ bits,
@@ -188,12 +267,118 @@ __global__ __launch_bounds__(WG) void k_quantize(int32_t quantizer, const void* 
     }
 }
 
+// Multiples of 8 that no other kernel takes: one wave per block in two passes
+// of vector accesses, the second of which finds the block in L2.  2^26 f32
+// in blocks of 4096 and 1000: 89 and 95 us; element by element 202 and 205.
+__global__ __launch_bounds__(WG) void k_quantize_vec(QuantArgs q, int64_t bs, const uint4* __restrict__ tables)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t lds[TABLE_BYTES];
+    stage_tables(lds, tables);
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int64_t wave = (int64_t)blockIdx.x * WAVES_PER_WG + uniform_u32(threadIdx.x / WAVE);
+    const int64_t nwaves = (int64_t)gridDim.x * WAVES_PER_WG;
+    for (int64_t b = wave; b < q.nblocks; b += nwaves) {
+        const int64_t base = b * bs;
+        const int64_t nvalid = max((int64_t)0, min(bs, q.size - base));
+        const int64_t nvec = nvalid / 8 * 8;
+        uint32_t am = 0;
+#pragma unroll 4
+        for (int64_t j = lane * 8; j < nvec; j += WAVE * 8) {
+            float x8[8];
+            load8_dt(q.x, q.x_dtype, base + j, x8);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) am = max(am, __float_as_uint(x8[t]) & 0x7FFFFFFFu);
+        }
+        for (int64_t j = nvec + lane; j < nvalid; j += WAVE)
+            am = max(am, __float_as_uint(load1(q.x, q.x_dtype, base + j)) & 0x7FFFFFFFu);
+        am = wave_max_u32(am);
+        const float scale = quant_scale(q, am);
+        if (lane == 0) store1(q.scales, q.scale_dtype, b, scale);  // scales.astype(scale_dtype) (adam8.py:186)
+        const bool fast = quant_fast(q, am, scale);
+        const float rs = 1.0f / scale;
+        for (int64_t j = lane * 8; j < nvec; j += WAVE * 8) {
+            const int64_t e0 = base + j;
+            float x8[8];
+            load8_dt(q.x, q.x_dtype, e0, x8);
+            const uint2 w = quant_code8(q, lds, x8, scale, rs, fast, e0);
+            __builtin_nontemporal_store((nt_u32x2){w.x, w.y}, (nt_u32x2*)(q.values + e0));
+        }
+        for (int64_t j = nvec + lane; j < bs; j += WAVE) {
+            const int64_t e = base + j;
+            const float xv = j < nvalid ? load1(q.x, q.x_dtype, e) : 0.0f;
+            q.values[e] = (uint8_t)quant_code(q, lds, xv, scale, rs, fast, e);
+        }
+    }
+}
+
+// Blocks of 2^lg elements, 8 .. 1024, x and values aligned: a wave per 1024
+// elements, lane l of its two chunks the eight from 8l, held in registers;
+// the absmax of several blocks are found at once within the wave, and a
+// chunk's registers take the wave's next tile as soon as it is coded.
+// Bound: HBM, with the LDS look-ups next.  2^26 f32 / bf16
+// in blocks of 256: 68 / 62 us (4.9 / 3.3 TB/s), of 1024: 65 / 48 us; a wave
+// per block in two element-wise passes 221 / 255 and 196 / 232.  Spans of a
+// run-time length with masks cost 7-20 %, and 2048-blocks in this form
+// spilled (190 us; k_quantize 69 / 62).
+__global__ __launch_bounds__(WG) void k_quantize_tile(QuantArgs q, int32_t lg, const uint4* __restrict__ tables)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t lds[TABLE_BYTES];
+    stage_tables(lds, tables);
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int64_t wave = (int64_t)blockIdx.x * WAVES_PER_WG + uniform_u32(threadIdx.x / WAVE);
+    const int64_t nwaves = (int64_t)gridDim.x * WAVES_PER_WG;
+    const int64_t total = q.nblocks << lg;
+    const int64_t ntiles = (total + TILE_SPAN - 1) / TILE_SPAN;
+    float r[2][8];
+    auto load_chunk = [&](int64_t tile, int j) {
+        const int64_t e0 = tile * TILE_SPAN + j * 512 + lane * 8;
+        if (e0 + 8 <= q.size) {
+            load8_dt(q.x, q.x_dtype, e0, r[j]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) r[j][t] = e0 + t < q.size ? load1(q.x, q.x_dtype, e0 + t) : 0.0f;
+        }
+    };
+    if (wave < ntiles) {
+        load_chunk(wave, 0);
+        load_chunk(wave, 1);
+    }
+    for (int64_t tile = wave; tile < ntiles; tile += nwaves) {
+        uint32_t am[2] = {0, 0};
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int t = 0; t < 8; ++t) am[j] = max(am[j], __float_as_uint(r[j][t]) & 0x7FFFFFFFu);
+        if (lg >= 10) {
+            am[0] = am[1] = wave_max_u32(max(am[0], am[1]));
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) am[j] = tile_max(am[j], lg);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int64_t e0 = tile * TILE_SPAN + j * 512 + lane * 8;
+            const float scale = quant_scale(q, am[j]);
+            const bool fast = quant_fast(q, am[j], scale);
+            if (e0 < total) {
+                const uint2 w = quant_code8(q, lds, r[j], scale, 1.0f / scale, fast, e0);
+                // nontemporal: the codes are not read again by this launch
+                __builtin_nontemporal_store((nt_u32x2){w.x, w.y}, (nt_u32x2*)(q.values + e0));
+                // scales.astype(scale_dtype) (adam8.py:186)
+                if ((e0 & ((1 << lg) - 1)) == 0) store1(q.scales, q.scale_dtype, e0 >> lg, scale);
+            }
+            if (tile + nwaves < ntiles) load_chunk(tile + nwaves, j);
+        }
+    }
+}
+
 // Standalone dequantize_blocks (adam8.py:190-204).  Vector path: each wave
 // takes 1024-element tiles, two at a time; lane l owns elements
 // 256k + 4l .. 256k + 4l + 3 (k = 0..3), so every code load reads 256
 // contiguous bytes and every store writes 1 KB (f32) or 512 B (bf16)
-// contiguous.  Requires a power-of-two block size (>= 4) and 4-byte aligned
-// codes / 16-byte (f32) or 8-byte (bf16) aligned output.
+// contiguous.  Requires a block size that is a multiple of 4 (POW2: a power of
+// two) and 4-byte aligned codes / 16-byte (f32) or 8-byte (bf16) aligned
+// output.
 __device__ __forceinline__ void dq_store4(void* out, int32_t out_dtype, int64_t e, const float (&o)[4])
 {
     // nontemporal: the launch does not read its output back
@@ -209,6 +394,7 @@ __device__ __forceinline__ void dq_store4(void* out, int32_t out_dtype, int64_t 
     }
 }
 
+template <bool POW2>
 __global__ __launch_bounds__(WG) void k_dequantize(int32_t quantizer, const uint8_t* __restrict__ values,
                                                    const void* __restrict__ scales, int32_t scale_dtype,
                                                    int64_t size, int64_t bs,
@@ -230,12 +416,18 @@ __global__ __launch_bounds__(WG) void k_dequantize(int32_t quantizer, const uint
         float s[T][4];
 #pragma unroll
         for (int u = 0; u < T; ++u) {
+            // other multiples of 4: the tile's block by one uniform division,
+            // the lane's from there in 32 bits
+            const int64_t b0 = POW2 ? 0 : (t0 + u) * 1024 / bs;
+            const uint32_t in0 = POW2 ? 0u : (uint32_t)((t0 + u) * 1024 - b0 * bs);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int64_t e = (t0 + u) * 1024 + k * 256 + lane * 4;
                 if (t0 + u < ntiles) {
                     w[u][k] = *(const uint32_t*)(values + e);
-                    s[u][k] = load1(scales, scale_dtype, e >> bs_log2);  // the 4 elements share a block (bs >= 4)
+                    // the 4 elements share a block (bs a multiple of 4)
+                    s[u][k] = load1(scales, scale_dtype,
+                                    POW2 ? e >> bs_log2 : b0 + (in0 + k * 256 + lane * 4) / (uint32_t)bs);
                 }
             }
         }
@@ -2703,11 +2895,31 @@ rf_status rf_blockwise_quantize(int32_t quantizer, const void* x, int32_t x_dtyp
     rf_status st = device_state(&ds);
     if (st != RF_OK) return st;
     const int64_t nb = nblocks_of(size, block_size);
+    unsigned grid = 1;
+    // Aligned buffers in blocks of other multiples of 8 than 2048: powers of
+    // two up to a wave's tile take the tile kernel, the rest the two vector
+    // passes; everything else k_quantize.
+    if (aligned(x, 16) && aligned(values, 8) && block_size % 8 == 0 && block_size != FAST_BS) {
+        const QuantArgs q{x, (uint8_t*)values, scales, bits, size, nb, key0, key1, quantizer, x_dtype, scale_dtype, sr};
+        if (block_size <= TILE_SPAN && (block_size & (block_size - 1)) == 0) {
+            const int32_t lg = 31 - __builtin_clz((unsigned)block_size);
+            st = worklist_grid((const void*)&k_quantize_tile, ds, (nb * block_size + TILE_SPAN - 1) / TILE_SPAN, &grid,
+                               8);
+            if (st != RF_OK) return st;
+            hipLaunchKernelGGL(k_quantize_tile, dim3(grid), dim3(WG), 0, (hipStream_t)stream, q, lg, ds->tables);
+        } else {
+            st = worklist_grid((const void*)&k_quantize_vec, ds, nb, &grid, 4);
+            if (st != RF_OK) return st;
+            hipLaunchKernelGGL(k_quantize_vec, dim3(grid), dim3(WG), 0, (hipStream_t)stream, q, (int64_t)block_size,
+                               ds->tables);
+        }
+        HIP_TRY(hipGetLastError());
+        return RF_OK;
+    }
     // One wave per block at a time, about 4 blocks per wave: on 2^30 f32
     // elements 0.968 ms, against 1.047 ms at 16 blocks per wave with ordinary
     // code stores and 1.023-1.027 ms with nontemporal ones; 2 per wave 0.971,
     // 1 per wave 0.986 (each workgroup stages its tables once).
-    unsigned grid = 1;
     st = worklist_grid((const void*)&k_quantize, ds, nb, &grid, 4);
     if (st != RF_OK) return st;
     const int32_t vec_ok = aligned(x, 16) && aligned(values, 8) && (!bits || aligned(bits, 16));
@@ -2734,7 +2946,7 @@ rf_status rf_blockwise_dequantize(int32_t quantizer, const void* values, const v
     const bool pow2 = block_size >= 4 && (block_size & (block_size - 1)) == 0;
     int32_t bs_log2 = 0;
     while (pow2 && (1 << bs_log2) < block_size) ++bs_log2;
-    const int32_t vec_ok = pow2 && aligned(values, 4) && aligned(out, out_dtype == RF_F32 ? 16 : 8);
+    const int32_t vec_ok = block_size % 4 == 0 && aligned(values, 4) && aligned(out, out_dtype == RF_F32 ? 16 : 8);
     // Vector path: one wave per two 1024-element tiles, every pair its own
     // wave (the workgroup stages only the 1 KB codebook): on 2^30 elements
     // 0.963 ms against 1.056 ms for a grid of 8 workgroups per CU walking the
@@ -2744,7 +2956,10 @@ rf_status rf_blockwise_dequantize(int32_t quantizer, const void* values, const v
     const int64_t wg_needed = std::max<int64_t>(1, (tiles + 2 * WAVES_PER_WG - 1) / (2 * WAVES_PER_WG));
     const int grid = (int)std::min<int64_t>(std::max<int64_t>(wg_needed, vec_ok ? 1 : (size + WG - 1) / WG),
                                             (int64_t)1 << 30);
-    hipLaunchKernelGGL(k_dequantize, dim3(grid), dim3(WG), 0, (hipStream_t)stream, quantizer,
+    // Blocks of 1000, 2^26 elements to f32 / bf16: 50 / 31 us, as for powers of
+    // two; element by element 253 / 235.
+    hipLaunchKernelGGL(pow2 ? &k_dequantize<true> : &k_dequantize<false>, dim3(grid), dim3(WG), 0,
+                       (hipStream_t)stream, quantizer,
                        (const uint8_t*)values, scales, scale_dtype, size, (int64_t)block_size, bs_log2, out_dtype,
                        out, ds->tables, vec_ok);
     HIP_TRY(hipGetLastError());
