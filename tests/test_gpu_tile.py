@@ -2,10 +2,10 @@
 CPU oracle: codes, scales and (exact=True) params bit for bit, default-mode
 params within one bf16 ulp.
 
-Block sizes at the edges of the kernel's three layouts (blocks of a power of
-two up to 1024 packed into 2048-element tiles; other multiples of 8 a wave
-each; blocks up to 8192 a workgroup each) and just outside them; leaves of
-whole tiles, of a partial last block and of a partial group of 8 elements;
+Block sizes at the edges of the kernel's layouts (powers of two up to 1024 in
+1024-element spans; other multiples of 8 below 1024 a wave each; up to 4096 a
+workgroup each) and just outside them; leaves of whole spans, of a partial
+last block and of a partial group of 8 elements;
 zero, tiny and non-finite blocks.
 """
 
