@@ -43,6 +43,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <exception>
 #include <string>
 #include <vector>
 
@@ -530,7 +531,8 @@ PyObject* py_apply_rows(PyObject*, PyObject* args)
 // tensors on one device, grads of the accumulator's shape whose dtype does
 // not promote the accumulator's.  None / MaskedNode accumulator leaves are
 // left out.  The result None means "not handled here": the Python walk then
-// converts, or raises the error.
+// converts, or raises the error.  So do leaves whose C++ accessors throw
+// (sparse tensors, wrappers without storage): no exception leaves the entry.
 struct AccumWalk {
     std::string rows;
     int device = -1;
@@ -549,7 +551,7 @@ bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w)
         const at::Tensor& ta = THPVariable_Unpack(a);
         rf_accum_leaf row{};
         row.acc_dtype = rf_dtype(ta.scalar_type());
-        if (row.acc_dtype < 0 || !ta.is_cuda() || !ta.is_contiguous()) return false;
+        if (row.acc_dtype < 0 || !ta.is_cuda() || ta.layout() != at::kStrided || !ta.is_contiguous()) return false;
         if (w.device < 0) w.device = ta.get_device();
         if (ta.get_device() != w.device) return false;
         row.acc = ta.data_ptr();
@@ -559,7 +561,8 @@ bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w)
             if (!THPVariable_Check(g)) return false;
             const at::Tensor& tg = THPVariable_Unpack(g);
             row.grad_dtype = rf_dtype(tg.scalar_type());
-            if (row.grad_dtype < 0 || !tg.is_cuda() || tg.get_device() != w.device || !tg.is_contiguous() ||
+            if (row.grad_dtype < 0 || !tg.is_cuda() || tg.get_device() != w.device ||
+                tg.layout() != at::kStrided || !tg.is_contiguous() ||
                 !tg.sizes().equals(ta.sizes()) || (row.grad_dtype != row.acc_dtype && row.acc_dtype != RF_F32))
                 return false;
             row.grad = tg.data_ptr();
@@ -575,7 +578,11 @@ bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w)
             PyObject* key = PyList_GET_ITEM(keys, k);
             PyObject* ca = PyDict_GetItemWithError(a, key);
             PyObject* cg = w.reset ? Py_None : PyDict_GetItemWithError(g, key);
-            ok = ca && cg && accum_walk(cg, ca, w);
+            try {
+                ok = ca && cg && accum_walk(cg, ca, w);
+            } catch (const std::exception&) {
+                ok = false;
+            }
         }
         Py_XDECREF(keys);
         PyErr_Clear();
@@ -598,7 +605,11 @@ PyObject* py_accum_rows(PyObject*, PyObject* args)
     if (!PyArg_ParseTuple(args, "OO", &g, &a)) return nullptr;
     AccumWalk w;
     w.reset = g == Py_None;
-    if (!accum_walk(g, a, w)) Py_RETURN_NONE;
+    try {
+        if (!accum_walk(g, a, w)) Py_RETURN_NONE;
+    } catch (const std::exception&) {
+        Py_RETURN_NONE;
+    }
     PyObject* rows = PyBytes_FromStringAndSize(w.rows.data(), (Py_ssize_t)w.rows.size());
     if (!rows) return nullptr;
     return Py_BuildValue("(Nnn)", rows, (Py_ssize_t)(w.rows.size() / sizeof(rf_accum_leaf)), (Py_ssize_t)w.device);

@@ -361,3 +361,24 @@ def test_magma_refuses_host_tensors():
     params = {"w": torch.zeros(4)}
     with pytest.raises((TypeError, ValueError)):
         tx.update({"w": torch.ones(4)}, tx.init(params), params)
+
+
+def test_native_accumulation_walk_leaves_storage_less_tensors_to_python():
+    """Tensors whose C++ accessors throw (a vmapped gradient has no storage)
+    are left to the Python walk; the exception does not end the process."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from rollfast_amd import _lib
+
+    host = _lib.pyhost()
+    got = []
+    with FakeTensorMode():
+        acc, grads = torch.empty(8, device="cuda"), torch.empty(3, 8, device="cuda")
+
+        def f(g):
+            for tree in (lambda x: x, lambda x: {"w": x}, lambda x: [(x,)]):
+                got.append(host.accum_rows(tree(g), tree(acc)))
+            return g
+
+        torch.vmap(f)(grads)
+    assert got == [None, None, None]
