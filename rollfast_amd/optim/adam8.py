@@ -460,11 +460,8 @@ def _one_minus(b) -> np.float32:
 
 def _bias_correction(b, count: int) -> np.float32:
     """``1.0 - b**count`` in f32 (adam8.py:338-339; f32 pow)."""
-    b32, c32 = _as_f32(b), np.float32(count)
-    if 0.0 <= b32 <= 1.0:  # nothing to warn of
-        return np.float32(1.0) - np.power(b32, c32)
     with np.errstate(all="ignore"):
-        return np.float32(1.0) - np.power(b32, c32)
+        return np.float32(1.0) - np.power(_as_f32(b), np.float32(count))
 
 
 # ------------------------------------------------------------ the engine ---

@@ -382,3 +382,10 @@ def test_native_accumulation_walk_leaves_storage_less_tensors_to_python():
 
         torch.vmap(f)(grads)
     assert got == [None, None, None]
+
+
+def test_bias_correction_ignores_the_callers_error_state():
+    """b**count underflows late in a run; that is no error, whatever the
+    caller's np.seterr says."""
+    with np.errstate(all="raise"):
+        assert A._bias_correction(0.9, 100_000) == 1.0
