@@ -107,7 +107,7 @@ def split(key, num: int = 2) -> np.ndarray:
     num = int(num)
     if num <= 16:
         k0, k1 = int(k[0]), int(k[1])
-        words = _native_split(k0, k1, num)
+        words = _native_split(k0, k1, num) if num > 0 else None
         if words is None:
             words = [_threefry_int(k0, k1, 0, i) for i in range(num)]
         return np.array(words, dtype=np.uint32).reshape(num, 2)

@@ -389,3 +389,12 @@ def test_bias_correction_ignores_the_callers_error_state():
     caller's np.seterr says."""
     with np.errstate(all="raise"):
         assert A._bias_correction(0.9, 100_000) == 1.0
+
+
+@pytest.mark.parametrize("num", [-2, -1, 0, 1, 16, 17])
+def test_split_counts(num):
+    """Every count gives what the Python integers give; none below zero."""
+    key = prng.PRNGKey(3)
+    words = prng.split(key, num)
+    assert words.shape == (max(num, 0), 2) and words.dtype == np.uint32
+    assert [tuple(w) for w in words] == [prng._threefry_int(int(key[0]), int(key[1]), 0, i) for i in range(num)]
