@@ -95,11 +95,11 @@ def _pyhost_job():
 def _sources_of(obj: str) -> list:
     """The source files an output is built from (headers included)."""
     inc = [os.path.join(REPO, "include", "rfadam8.h")]
-    dev = [os.path.join(CSRC, "rf_device.h"), os.path.join(CSRC, "rf_tables.h")]
+    dev = [os.path.join(CSRC, name) for name in ("rf_device.h", "rf_tile.h", "rf_tables.h")]
     if obj.endswith("rf_host.o"):
         return [HOST_SRC, *dev, *inc]
     if os.path.basename(obj).startswith("rf_tile"):
-        return [TILE_SRC, os.path.join(CSRC, "rf_tile.h"), *dev, *inc]
+        return [TILE_SRC, *dev, *inc]
     if obj.endswith(".o"):
         return [INST_SRC, *dev, *inc]
     return [PYHOST_SRC, *inc, __file__]
