@@ -11,6 +11,7 @@ from rollfast_amd import build
 
 def _included(path, seen):
     """The repository's own files that `path` includes, itself among them."""
+    path = os.path.normpath(path)
     if path in seen:
         return seen
     seen.add(path)
