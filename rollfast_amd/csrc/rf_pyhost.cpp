@@ -608,6 +608,7 @@ PyObject* py_accum_rows(PyObject*, PyObject* args)
     try {
         if (!accum_walk(g, a, w)) Py_RETURN_NONE;
     } catch (const std::exception&) {
+        PyErr_Clear();  // a leaf's own Python error: the Python walk meets and raises it again
         Py_RETURN_NONE;
     }
     PyObject* rows = PyBytes_FromStringAndSize(w.rows.data(), (Py_ssize_t)w.rows.size());

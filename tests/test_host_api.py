@@ -384,6 +384,32 @@ def test_native_accumulation_walk_leaves_storage_less_tensors_to_python():
     assert got == [None, None, None]
 
 
+@pytest.mark.parametrize("tree", [lambda x: x, lambda x: [x], lambda x: {"w": x}, lambda x: {"w": (x,)}],
+                         ids=["leaf", "list", "dict", "dict of tuple"])
+def test_native_accumulation_walk_keeps_a_leafs_own_error(tree):
+    """A leaf whose layout query raises (a wrapper subclass that answers it
+    itself): the native walk returns None with no error set, and the
+    accumulation raises the leaf's own error."""
+    from rollfast_amd import _lib
+
+    class Odd(torch.Tensor):
+        @staticmethod
+        def __new__(cls):
+            return torch.Tensor._make_wrapper_subclass(cls, (8,), dtype=torch.float32, device="cuda",
+                                                       dispatch_sizes_strides_policy="strides")
+
+        @classmethod
+        def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+            raise LookupError("the leaf's own error")
+
+    x = tree(Odd())
+    assert _lib.pyhost().accum_rows(x, x) is None
+    assert _lib.pyhost().accum_rows(None, x) is None
+    ms = rf.MultiSteps(rf.adamw8(1e-3), every_k_schedule=2)
+    with pytest.raises(LookupError, match="own error"):
+        ms.update._accumulate(x, x, _lib.RF_ACC_SUM, 0)
+
+
 def test_bias_correction_ignores_the_callers_error_state():
     """b**count underflows late in a run; that is no error, whatever the
     caller's np.seterr says."""
