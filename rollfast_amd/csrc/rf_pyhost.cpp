@@ -531,8 +531,10 @@ PyObject* py_apply_rows(PyObject*, PyObject* args)
 // tensors on one device, grads of the accumulator's shape whose dtype does
 // not promote the accumulator's.  None / MaskedNode accumulator leaves are
 // left out.  The result None means "not handled here": the Python walk then
-// converts, or raises the error.  So do leaves whose C++ accessors throw
-// (sparse tensors, wrappers without storage): no exception leaves the entry.
+// converts, or raises the error.  So do tensor subclasses other than
+// torch.nn.Parameter, whose Python overrides (device, layout, data pointer)
+// the C++ accessors would pass by, and leaves whose accessors throw (sparse
+// tensors, wrappers without storage): no exception leaves the entry.
 struct AccumWalk {
     std::string rows;
     int device = -1;
@@ -548,6 +550,7 @@ bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w)
 {
     if (is_aux(a)) return w.reset || is_grad_leaf(g);
     if (THPVariable_Check(a)) {
+        if (!THPVariable_CheckExact(a) || (!w.reset && !THPVariable_CheckExact(g))) return false;
         const at::Tensor& ta = THPVariable_Unpack(a);
         rf_accum_leaf row{};
         row.acc_dtype = rf_dtype(ta.scalar_type());
@@ -558,7 +561,6 @@ bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w)
         row.size = ta.numel();
         row.grad_dtype = row.acc_dtype;
         if (!w.reset) {
-            if (!THPVariable_Check(g)) return false;
             const at::Tensor& tg = THPVariable_Unpack(g);
             row.grad_dtype = rf_dtype(tg.scalar_type());
             if (row.grad_dtype < 0 || !tg.is_cuda() || tg.get_device() != w.device ||

@@ -410,6 +410,37 @@ def test_native_accumulation_walk_keeps_a_leafs_own_error(tree):
         ms.update._accumulate(x, x, _lib.RF_ACC_SUM, 0)
 
 
+def test_native_accumulation_walk_leaves_subclasses_to_python():
+    """A subclass may answer data_ptr() and the layout queries itself: the
+    native walk, which would read the wrapper's own (null) storage, leaves it
+    to the Python walk, as accumulator and as gradient."""
+    from rollfast_amd import _lib
+
+    asked = []
+
+    class Inner(torch.Tensor):
+        @staticmethod
+        def __new__(cls):
+            return torch.Tensor._make_wrapper_subclass(cls, (8,), dtype=torch.float32, device="cuda")
+
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            asked.append(getattr(func, "__name__", func))
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+        @classmethod
+        def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+            raise AssertionError(func)
+
+    host = _lib.pyhost()
+    for x in (Inner(), [Inner()], {"w": Inner()}):
+        assert host.accum_rows(x, x) is None and host.accum_rows(None, x) is None
+    ms = rf.MultiSteps(rf.adamw8(1e-3), every_k_schedule=2)
+    with pytest.raises((RuntimeError, ValueError, AssertionError)):  # no GPU, or the null pointer refused
+        ms.update._accumulate(Inner(), Inner(), _lib.RF_ACC_SUM, 0)
+    assert "data_ptr" in asked
+
+
 def test_bias_correction_ignores_the_callers_error_state():
     """b**count underflows late in a run; that is no error, whatever the
     caller's np.seterr says."""
