@@ -57,9 +57,10 @@ def _compile_jobs():
     jobs = [([HIPCC, *FLAGS, *inc, "-c", HOST_SRC, "-o", os.path.join(OBJ_DIR, "rf_host.o")],
              os.path.join(OBJ_DIR, "rf_host.o"))]
     for a, m, e in VARIANTS:
-        obj = os.path.join(OBJ_DIR, f"rf_adam8_a{a}_m{m}_e{e}.o")
-        defs = [f"-DRFI_APPLY={a}", f"-DRFI_MSR={m}", f"-DRFI_EXACT={e}"]
-        jobs.append(([HIPCC, *FLAGS, *inc, *defs, "-c", INST_SRC, "-o", obj], obj))
+        for gen, kernel in enumerate(("adam8", "gen")):
+            obj = os.path.join(OBJ_DIR, f"rf_{kernel}_a{a}_m{m}_e{e}.o")
+            defs = [f"-DRFI_APPLY={a}", f"-DRFI_MSR={m}", f"-DRFI_EXACT={e}", f"-DRFI_GEN={gen}"]
+            jobs.append(([HIPCC, *FLAGS, *inc, *defs, "-c", INST_SRC, "-o", obj], obj))
     for a, m, e in VARIANTS:
         obj = os.path.join(OBJ_DIR, f"rf_tile_a{a}_m{m}_e{e}.o")
         defs = [f"-DRFI_APPLY={a}", f"-DRFI_MSR={m}", f"-DRFI_EXACT={e}"]
@@ -117,7 +118,7 @@ def build(verbose: bool = False, jobs: int | None = None, incremental: bool = Fa
     the path of the built ``.so``.  ``incremental``: recompile only the
     objects older than their sources."""
     os.makedirs(OBJ_DIR, exist_ok=True)
-    max_par = jobs or min(2 * len(VARIANTS) + 1, max(1, os.cpu_count() or 1))
+    max_par = jobs or min(3 * len(VARIANTS) + 1, max(1, os.cpu_count() or 1))
     # the moment-SR objects compile longest: first, so that none runs alone at the end
     pending = sorted(_compile_jobs(), key=lambda job: ("_m1_" not in job[1], "tile" in job[1])) + [_pyhost_job()]
     if incremental:

@@ -2350,8 +2350,8 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(RF_STEP_WAVE
         if (bid < gw) {
             // the generic units do not use the per-wave tables: their
             // workgroup absmax words take the first of them
-            gen_list<APPLY, MSR, PSR, NEST, EXACT, false>(leaves, h.gsegs, h.gunits, h, tables, lds,
-                                                          (uint32_t*)&wtab[0][0], bid, gw);
+            gen_list<APPLY, MSR, PSR, NEST, EXACT, false, true>(leaves, h.gsegs, h.gunits, h, tables, lds,
+                                                                (uint32_t*)&wtab[0][0], bid, gw);
             return;
         }
         bid -= gw;
@@ -2510,6 +2510,11 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(RF_STEP_WAVE
 // blocks (a workgroup each; two passes, literal requantization), then the
 // leaves with unquantized (fallback) moments (a wave per unit).  Dtypes are
 // read per leaf.
+// TEAM: an instance for lists that hold KIND_QTEAM units (rf_tile.h).  Their
+// registers and, with moment SR, their search tables cost the two-pass units
+// of a list without them: with moment SR 165 VGPRs and 30 KB to stage for 118
+// to 137 and 22, and 512 blocks of 1000 elements, all SR, 21.7 us for 17.4
+// (2,048 of 64: 31.2 for 20.9).
 // VEC_ONLY: an instance for lists of full-chunk fallback units only (the
 // full-precision AdamW trees).  Without the other unit kinds its plain
 // instances take 126-127 VGPRs (4 waves per SIMD) as the compiler schedules
@@ -2524,8 +2529,9 @@ constexpr int GEN_WAVES_PER_EU = (VEC_ONLY || MSR || PSR || NEST) ? 1 : 4;
 // The generic list's units over workgroups bid = 0 .. nbid - 1 of a launch:
 // the generic kernel's whole grid, or the leading workgroups of a fast
 // launch the list rides along with (k_adam8, KHp.gsegs).  `lds` holds at
-// least TABLE_BYTES (SEARCH_BYTES with moment SR); `red` is 8 words of LDS.
-template <bool APPLY, bool MSR, bool PSR, bool NEST, bool EXACT, bool VEC_ONLY>
+// least TABLE_BYTES (SEARCH_BYTES with TEAM and moment SR); `red` is 8 words
+// of LDS.
+template <bool APPLY, bool MSR, bool PSR, bool NEST, bool EXACT, bool VEC_ONLY, bool TEAM>
 __device__ __forceinline__ void gen_list(const rf_adam8_leaf* __restrict__ leaves, const Seg* __restrict__ segs,
                                          int64_t total_units, const KHp& h, const uint4* __restrict__ tables,
                                          uint8_t* lds, uint32_t* red, uint32_t bid, uint32_t nbid)
@@ -2535,7 +2541,8 @@ __device__ __forceinline__ void gen_list(const rf_adam8_leaf* __restrict__ leave
     // tables (null: the list has no quantized units).  The others
     // (element-wise units of small leaves) start at once.
     const int64_t nlead = VEC_ONLY ? 0 : segs[0].lead;
-    if (!VEC_ONLY && tables && (int64_t)bid < nlead) stage_tables<MSR ? SEARCH_BYTES : TABLE_BYTES>(lds, tables);
+    if (!VEC_ONLY && tables && (int64_t)bid < nlead)
+        stage_tables<TEAM && MSR ? SEARCH_BYTES : TABLE_BYTES>(lds, tables);
 
     const int64_t wave = (int64_t)bid * WAVES_PER_WG + uniform_u32(threadIdx.x / WAVE);
     const int64_t nwaves = (int64_t)nbid * WAVES_PER_WG;
@@ -2563,7 +2570,6 @@ __device__ __forceinline__ void gen_list(const rf_adam8_leaf* __restrict__ leave
     // the full ones of a short list), a workgroup each; then the rest a wave each, handed out
     // from the last waves down so that the workgroups of the first phase
     // take none when the workgroups cover every unit.
-    TileSlot sl[2];
     for (int64_t q = bid; q < nlead; q += nbid) {
         s = seek_seg(segs, nseg, s, q);
         const Seg sg = segs[s];
@@ -2571,15 +2577,20 @@ __device__ __forceinline__ void gen_list(const rf_adam8_leaf* __restrict__ leave
             cur_leaf = sg.leaf;
             L = leaves[cur_leaf];
             group_hparams(hl, h, L);
-            flr_setup(hl);
+            if constexpr (TEAM) flr_setup(hl);
             leaf_context<false>(c, L, hl, MSR, PSR);
             if (h.mpart) c.mbase = h.msegs[cur_leaf].unit_start;
         }
         const int64_t blk = sg.first + (q - sg.unit_start);
-        if (sg.kind == KIND_QTEAM)
-            unit_tile<DT_ANY, APPLY, MSR, PSR, EXACT, false, 1>(c, L, hl, NEST, true, team_span(L, blk), sl, false,
-                                                                TileSpan{}, red);
-        else unit_qgen_wg<APPLY, MSR, PSR, NEST, EXACT>(c, L, blk, hl, red);
+        if constexpr (TEAM) {
+            if (sg.kind == KIND_QTEAM) {
+                TileSlot sl[2];
+                unit_tile<DT_ANY, APPLY, MSR, PSR, EXACT, false, 1>(c, L, hl, NEST, true, team_span(L, blk), sl, false,
+                                                                    TileSpan{}, red);
+                continue;
+            }
+        }
+        unit_qgen_wg<APPLY, MSR, PSR, NEST, EXACT>(c, L, blk, hl, red);
     }
     for (int64_t u = nlead + (nwaves - 1 - wave); u < total_units; u += nwaves) {
         s = seek_seg(segs, nseg, s, u);
@@ -2603,16 +2614,16 @@ __device__ __forceinline__ void gen_list(const rf_adam8_leaf* __restrict__ leave
     }
 }
 
-template <bool APPLY, bool MSR, bool PSR, bool NEST, bool EXACT, bool VEC_ONLY = false>
+template <bool APPLY, bool MSR, bool PSR, bool NEST, bool EXACT, bool VEC_ONLY = false, bool TEAM = false>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(GEN_WAVES_PER_EU<MSR, PSR, NEST, VEC_ONLY>)))
 void k_adam8_gen(const rf_adam8_leaf* __restrict__ leaves,
                                                   const Seg* __restrict__ segs, int64_t total_units, KHp h,
                                                   const uint4* __restrict__ tables)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[VEC_ONLY ? 16 : MSR ? SEARCH_BYTES : TABLE_BYTES];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[VEC_ONLY ? 16 : TEAM && MSR ? SEARCH_BYTES : TABLE_BYTES];
     __shared__ uint32_t red[2 * WAVES_PER_WG];  // absmax bits of a workgroup's block, per wave
-    gen_list<APPLY, MSR, PSR, NEST, EXACT, VEC_ONLY>(leaves, segs, total_units, h, tables, lds, red, blockIdx.x,
-                                                     gridDim.x);
+    gen_list<APPLY, MSR, PSR, NEST, EXACT, VEC_ONLY, TEAM>(leaves, segs, total_units, h, tables, lds, red, blockIdx.x,
+                                                           gridDim.x);
 }
 
 }  // namespace rf

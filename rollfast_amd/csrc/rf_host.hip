@@ -47,6 +47,15 @@ adam_kernel_t rf_pick_adam8_a1_m0_e0(int dtype_combo, bool psr, bool nest);
 adam_kernel_t rf_pick_adam8_a1_m0_e1(int dtype_combo, bool psr, bool nest);
 adam_kernel_t rf_pick_adam8_a1_m1_e0(int dtype_combo, bool psr, bool nest);
 adam_kernel_t rf_pick_adam8_a1_m1_e1(int dtype_combo, bool psr, bool nest);
+// Instances of the generic kernel (rf_adam8_inst.hip).
+adam_kernel_t rf_pick_gen_a0_m0_e0(int combo, bool psr, bool nest);
+adam_kernel_t rf_pick_gen_a0_m0_e1(int combo, bool psr, bool nest);
+adam_kernel_t rf_pick_gen_a0_m1_e0(int combo, bool psr, bool nest);
+adam_kernel_t rf_pick_gen_a0_m1_e1(int combo, bool psr, bool nest);
+adam_kernel_t rf_pick_gen_a1_m0_e0(int combo, bool psr, bool nest);
+adam_kernel_t rf_pick_gen_a1_m0_e1(int combo, bool psr, bool nest);
+adam_kernel_t rf_pick_gen_a1_m1_e0(int combo, bool psr, bool nest);
+adam_kernel_t rf_pick_gen_a1_m1_e1(int combo, bool psr, bool nest);
 // Instances of the tile kernel (rf_tile_inst.hip).
 adam_kernel_t rf_pick_tile_a0_m0_e0(bool bf16, bool psr);
 adam_kernel_t rf_pick_tile_a0_m0_e1(bool bf16, bool psr);
@@ -845,8 +854,25 @@ constexpr StepShape STEP_SHAPE_STREAM = {2, 8};
 constexpr StepShape STEP_SHAPE_HEAVY = {4, 16};
 // The tile kernel's units are half as long: the streaming shape in elements.
 // A 202 M-parameter bf16 layer in blocks of 256, runs of 2 and 16 or 32
-// units per wave 437 us, runs of 4 and 16 443 us.
+// units per wave 437 us, runs of 4 and 16 443 us.  Lists of at most
+// a chip-full of waves are handed out one unit at a time instead, so that no
+// wave takes a second unit while others have none: 2,048 spans of 1024, all
+// SR 31.9 us for 42.0, bf16 nearest 16.9 for 18.4; with 6,144 spans f32
+// nearest runs of one took 35.6 us for 34.1.
 constexpr StepShape STEP_SHAPE_TILE = {2, 16};
+// Short lists of other block sizes run in the generic list, a workgroup per
+// block in two passes (blocks up to a span) or one (up to 2048), instead of
+// the tile kernel: one launch for the tree, and 256 lanes on a block's
+// latencies and draws where the tile kernel has a wave's 16 elements per
+// lane.  The line is a number of blocks that falls with their size: 8 per
+// CU up to 128 elements, 6 up to 512, 4 beyond; a list of several sizes
+// counts each by its own.  One GPU, kernels only, generic / tile one unit at
+// a time, bf16 nearest and all SR: 1,024 blocks of 64 11.4 / 15.8 and 13.5 /
+// 28.0 us, 3,072 17.4 / 15.6 and 27.5 / 28.1; 512 blocks of 256 10.4 / 16.0
+// and 15.5 / 28.4, 2,048 17.3 / 15.3 and 32.7 / 28.6; 512 blocks of 1000
+// 11.2 / 15.3 and 17.3 / 27.9, 1,536 19.7 / 17.0 and 35.2 / 31.2.
+constexpr int64_t SHORT_WEIGHT_PER_CU = 24;
+constexpr int64_t short_weight(int64_t bs) { return bs > 512 ? 6 : bs > 128 ? 4 : 3; }
 // Short lists of full 2048-blocks run in the generic list instead of
 // k_adam8, a workgroup per block: one launch for the tree whatever its
 // dtypes, and four waves on a block's memory latencies and random draws
@@ -1694,9 +1720,10 @@ inline bool valid_dtype(int32_t d) { return d == RF_F32 || d == RF_BF16 || d == 
 // ---- kernel selection ----
 // The fast kernel's instances: dtype_combo = 2*(param is bf16) + (grad is bf16)
 // for f32/bf16 params and grads, COMBO_F16 for f16 params and grads; -1 (the
-// generic kernel) for the other mixes, VEC_COMBO (its instance without the
-// element-wise and quantized unit code) for a generic list that holds
-// full-chunk fallback units only.
+// generic kernel) for the other mixes, GEN_TEAM_COMBO (its instance with
+// rf_tile.h's units) for a generic list that holds KIND_QTEAM units,
+// VEC_COMBO (its instance without the element-wise and quantized unit code)
+// for one that holds full-chunk fallback units only.
 constexpr int COMBO_F16 = 4;
 constexpr int GEN_LIST = 5;    // the generic kernel's work list
 constexpr int GEN_TAIL = 6;    // build space: its fallback units, appended after its quantized ones
@@ -1708,6 +1735,8 @@ constexpr int N_LISTS = 10;
 constexpr int VEC_COMBO = -2;  // a generic list of full-chunk fallback units only
 constexpr int TILE_COMBO = -3;       // the tile list (k_adam8_tile)
 constexpr int TILE_BF16_COMBO = -4;  // the same where every leaf has bf16 params and grads
+constexpr int GEN_TEAM_COMBO = -5;   // a generic list with KIND_QTEAM units
+inline bool is_gen(int combo) { return combo == -1 || combo == GEN_TEAM_COMBO; }
 inline bool is_tile(int combo) { return combo == TILE_COMBO || combo == TILE_BF16_COMBO; }
 // Largest block the tile kernel holds in registers (a span per wave of a workgroup).
 constexpr int64_t TILE_MAX_BS = WAVES_PER_WG * TILE_SPAN;
@@ -1724,6 +1753,14 @@ adam_kernel_t pick_adam_kernel(bool apply, bool msr, bool psr, bool nest, bool e
         return exact ? rf_pick_tile_a0_m0_e1(b, false) : rf_pick_tile_a0_m0_e0(b, false);
     }
     if (combo == VEC_COMBO) msr = false;  // fallback units have no codes to round
+    if (is_gen(combo) || combo == VEC_COMBO) {
+        if (apply) {
+            if (msr) return exact ? rf_pick_gen_a1_m1_e1(combo, psr, nest) : rf_pick_gen_a1_m1_e0(combo, psr, nest);
+            return exact ? rf_pick_gen_a1_m0_e1(combo, psr, nest) : rf_pick_gen_a1_m0_e0(combo, psr, nest);
+        }
+        if (msr) return exact ? rf_pick_gen_a0_m1_e1(combo, false, nest) : rf_pick_gen_a0_m1_e0(combo, false, nest);
+        return exact ? rf_pick_gen_a0_m0_e1(combo, false, nest) : rf_pick_gen_a0_m0_e0(combo, false, nest);
+    }
     if (apply) {
         if (msr) return exact ? rf_pick_adam8_a1_m1_e1(combo, psr, nest) : rf_pick_adam8_a1_m1_e0(combo, psr, nest);
         return exact ? rf_pick_adam8_a1_m0_e1(combo, psr, nest) : rf_pick_adam8_a1_m0_e0(combo, psr, nest);
@@ -1972,8 +2009,8 @@ struct WorkLists {
 
 // merge_max: lists of at most this many full 2048-blocks get the merged form
 // too; merged_only: these get no other.
-rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_t apply, int64_t merge_max,
-                           bool merged_only, WorkLists& w)
+rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_t apply, int32_t num_cus,
+                           int64_t merge_max, bool merged_only, WorkLists& w)
 {
     rf_status st = RF_OK;
     std::vector<Seg>* gsegs = w.gsegs;
@@ -1993,12 +2030,28 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
     };
     std::vector<uint8_t>& vecs = w.vecs;
     vecs.clear();
+    // Leaves the tile kernel can take: aligned, blocks of a multiple of 8
+    // elements that a workgroup's registers hold, and (2048) no k_adam8
+    // instance of their dtypes.
+    auto tile_leaf = [&](int32_t i) {
+        const rf_adam8_leaf& L = leaves[i];
+        return L.moment_kind == RF_MOMENT_QUANTIZED && vecs[i] && L.block_size % 8 == 0 &&
+               L.block_size <= TILE_MAX_BS && (L.block_size != FAST_BS || dtype_combo(L) < 0);
+    };
+    const int64_t short_max = SHORT_WEIGHT_PER_CU * num_cus;
+    int64_t tile_weight = 0;
     for (int32_t i = 0; i < n_leaves; ++i) {
         const rf_adam8_leaf& L = leaves[i];
         st = validate_leaf(L, i, apply);
         if (st != RF_OK) return st;
-        const bool vec = leaf_vec_ok(L, apply);
-        vecs.push_back(vec ? 1 : 0);
+        vecs.push_back(leaf_vec_ok(L, apply) ? 1 : 0);
+        if (tile_leaf(i) && tile_weight <= short_max)
+            tile_weight += short_weight(L.block_size) * std::min<int64_t>(nblocks_of(L.size, L.block_size), short_max);
+    }
+    const bool tile_short = tile_weight <= short_max;
+    for (int32_t i = 0; i < n_leaves; ++i) {
+        const rf_adam8_leaf& L = leaves[i];
+        const bool vec = vecs[i] != 0;
         // Full aligned 2048-blocks go to the fast kernel of their dtype
         // combination; everything else to the generic kernel (GEN_LIST).
         const int combo = dtype_combo(L);
@@ -2009,13 +2062,16 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
                 const int64_t nfull = L.size / bs;
                 add(i, combo, KIND_QFAST, 0, nfull);
                 add(i, GEN_LIST, KIND_QTEAM, nfull, nb - nfull);
-            } else if (vec && bs % 8 == 0 && bs <= TILE_MAX_BS) {
+            } else if (tile_leaf(i) && tile_short && bs <= FAST_BS) {
+                add(i, GEN_LIST, bs <= TILE_SPAN ? KIND_QGEN : KIND_QTEAM, 0, nb);
+            } else if (tile_leaf(i)) {
                 // Aligned leaves of other block sizes (and of 2048 with a
                 // dtype mix that has no k_adam8 instance): the tile kernel.
                 // A 202 M-parameter bf16 layer in blocks of 256: 437 us,
                 // 6.63 ms in the generic kernel's workgroup per block.
                 // Blocks that are not a multiple of 8 elements, or beyond
-                // the registers of a workgroup, stay there.
+                // the registers of a workgroup, stay there, and so do short
+                // lists (SHORT_WEIGHT_PER_CU).
                 tile_blocks += nb;
                 tile_bf16 &= combo == 3;
                 if (bs < TILE_SPAN && (bs & (bs - 1)) == 0)
@@ -2094,15 +2150,18 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
         const bool plain = combo != MERGED_LIST;                        // in `groups`
         const bool in_merged = combo == TILE_LIST || combo == MERGED_LIST;  // in `merged`
         if (merged_only && gunits[MERGED_LIST] > 0 && !in_merged) continue;
-        bool quant = !generic, vec_only = generic;
+        bool quant = !generic, vec_only = generic, team = false;
         for (const Seg& sg : gsegs[combo]) {
             quant |= sg.kind == KIND_QGEN || sg.kind == KIND_QTEAM;
+            team |= sg.kind == KIND_QTEAM;
             vec_only &= sg.kind == KIND_FALLBACK_VEC;
         }
         const int kc = combo == TILE_LIST ? (tile_bf16 ? TILE_BF16_COMBO : TILE_COMBO)
                        : !generic         ? combo
-                                          : (vec_only ? VEC_COMBO : -1);
-        const int64_t lead = kc == -1 ? gen_lead + (plain ? 0 : nfast) : is_tile(kc) ? tile_lead : 0;
+                       : vec_only         ? VEC_COMBO
+                       : team             ? GEN_TEAM_COMBO
+                                          : -1;
+        const int64_t lead = is_gen(kc) ? gen_lead + (plain ? 0 : nfast) : is_tile(kc) ? tile_lead : 0;
         const PlanGroup group = {kc, (int64_t)segs.size(), gunits[combo], quant, lead};
         if (plain) {
             groups.push_back(group);
@@ -2261,7 +2320,7 @@ rf_status rf_adam8_plan_create(const rf_adam8_leaf* leaves, int32_t n_leaves, in
     rf_status st = device_state(&ds);
     if (st != RF_OK) return st;
     WorkLists w;
-    st = build_work_lists(leaves, n_leaves, apply, MERGE_BLOCKS_PER_CU_HEAVY * ds->num_cus, false, w);
+    st = build_work_lists(leaves, n_leaves, apply, ds->num_cus, MERGE_BLOCKS_PER_CU_HEAVY * ds->num_cus, false, w);
     if (st != RF_OK) return st;
     std::vector<Seg>& segs = w.segs;
     std::vector<Seg>& nsegs = w.nsegs;
@@ -2415,7 +2474,7 @@ void find_carrier(const std::vector<PlanGroup>& groups, bool msr, const PlanGrou
 {
     *gen = *carrier = nullptr;
     for (const PlanGroup& g : groups) {
-        if (g.combo == -1) *gen = &g;
+        if (is_gen(g.combo)) *gen = &g;
         if (g.combo == 3) *carrier = &g;
     }
     if (!*gen || msr) *carrier = nullptr;
@@ -2435,7 +2494,7 @@ int64_t step_grid(const DevState* ds, int occ, const PlanGroup& g, int32_t run, 
         std::min(wg_needed, (units + (int64_t)WAVES_PER_WG * per_wave - 1) / ((int64_t)WAVES_PER_WG * per_wave));
     int64_t grid = std::max<int64_t>(1, std::max(std::min(wg_needed, wg_resident), wg_spread));
     const int64_t wg_each = g.lead + (g.units - g.lead + WAVES_PER_WG - 1) / WAVES_PER_WG;
-    if (g.combo == -1 && wg_each <= GEN_WAVE_PER_UNIT_MAX_ROUNDS * wg_resident) {
+    if (is_gen(g.combo) && wg_each <= GEN_WAVE_PER_UNIT_MAX_ROUNDS * wg_resident) {
         // Mixed generic lists: a workgroup per leading quantized unit, then
         // a wave per unit.  These units are latency-bound (a partial block,
         // a leaf's tail), so the workgroups beyond a chip-full queue behind
@@ -2576,6 +2635,7 @@ rf_status plan_launch(const rf_adam8_plan* plan, const rf_adam8_leaf* d_leaves, 
         const bool streaming = plan->apply && !msr && !psr && !(f & RF_EXACT);
         const StepShape shape = is_tile(g.combo) ? STEP_SHAPE_TILE : streaming ? STEP_SHAPE_STREAM : STEP_SHAPE_HEAVY;
         k.run = g.combo < 0 && !is_tile(g.combo) ? 1 : shape.run;
+        if (is_tile(g.combo) && g.units - g.lead <= (int64_t)ds->num_cus * occ * WAVES_PER_WG) k.run = 1;
         // f32 updates (update-only launches) and f32 params are stored on
         // whole cache lines; nontemporally from UPD_NT_MIN_BLOCKS_PER_CU
         // blocks per CU on.  Three store forms on one GPU (old half-line
@@ -2811,7 +2871,8 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     std::lock_guard<std::mutex> order(ds->noalloc_mu);
     // Host-side lists in per-thread buffers that keep their capacity.
     thread_local WorkLists w;
-    st = build_work_lists(leaves, n_leaves, apply, merge_max(ds, light_leaves(leaves, n_leaves), hp->flags, apply), true, w);
+    st = build_work_lists(leaves, n_leaves, apply, ds->num_cus,
+                          merge_max(ds, light_leaves(leaves, n_leaves), hp->flags, apply), true, w);
     if (st != RF_OK) return st;
 
     // Scratch layout: what the host stages (leaf table, group table, step and

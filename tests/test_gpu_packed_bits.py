@@ -43,14 +43,14 @@ def _key(k):
     return tuple(int(v) for v in k)
 
 
-def _run_packed(spec, *, steps, msr, psr, seed=0, wd=0.01, lr=1e-3):
+def _run_packed(spec, *, steps, msr, psr, seed=0, wd=0.01, lr=1e-3, block_size=2048):
     import torch
 
     import rollfast_amd as rf
 
     host_params, params = _build(spec, seed)
     tx = rf.adamw8(learning_rate=lr, weight_decay=wd, stochastic_rounding=msr, exact=True, key=rf.prng.PRNGKey(7),
-                   sr_bits="packed")
+                   sr_bits="packed", block_size=block_size)
     state = tx.init(params)
     n = len(spec)
     for step in range(steps):
@@ -100,12 +100,10 @@ def test_packed_moment_sr_fill_blocks_one_big_leaf():
 
 
 def test_packed_both_roundings_block_4096():
-    """Blocks of 4096 (the generic kernel, a workgroup per block, literal
-    coding) with both roundings from the packed source."""
-    import rollfast_amd as rf  # noqa: F401
-
+    """Blocks of 4096 (a workgroup per block, 1024 elements per wave), whole
+    and partial, with both roundings from the packed source."""
     spec = [((3, 5000), "bf16", "bf16"), ((9000,), "bf16", "f32"), ((64, 2048), "bf16", "bf16")]
-    _run_packed(spec, steps=2, msr=True, psr=True)
+    _run_packed(spec, steps=2, msr=True, psr=True, block_size=4096)
 
 
 def test_packed_optax_form_equals_fused():
