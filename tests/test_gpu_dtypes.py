@@ -82,7 +82,7 @@ def _tree_spec():
             ((3, 2048), "bf16", "bf16"), ((2, 2048), "f32", "f32"), ((900,), "f16", "f16"), ((300,), "f16", "f32")]
 
 
-def _adamw8_tree_run(*, scale_dtype, fallback, exact, steps=3, psr=False, clip=None):
+def _adamw8_tree_run(*, scale_dtype, fallback, exact, steps=3, psr=False, clip=None, block_size=2048):
     import torch
 
     rf = _rf()
@@ -92,7 +92,7 @@ def _adamw8_tree_run(*, scale_dtype, fallback, exact, steps=3, psr=False, clip=N
     params = {f"l{i}": to_device(h, pd).reshape(s) for i, (h, (s, pd, _)) in enumerate(zip(host_p, spec))}
     tdt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
     tx = rf.adamw8(learning_rate=1e-3, weight_decay=0.01, min_size=1024, exact=exact,
-                   scale_dtype=tdt[scale_dtype], fallback_dtype=tdt[fallback])
+                   scale_dtype=tdt[scale_dtype], fallback_dtype=tdt[fallback], block_size=block_size)
     state = tx.init(params)
     leaves = []
     for i, (s, pd, gd) in enumerate(spec):
@@ -100,7 +100,7 @@ def _adamw8_tree_run(*, scale_dtype, fallback, exact, steps=3, psr=False, clip=N
         L = {"pdtype": pd, "gdtype": gd, "size": int(np.prod(s)), "param": None}
         if isinstance(m, rf.QuantizedBlocks):
             assert m.scales.dtype == tdt[scale_dtype]
-            L.update(kind="quant", block_size=2048, mu=to_host(m.values).copy(), nu=to_host(v.values).copy(),
+            L.update(kind="quant", block_size=block_size, mu=to_host(m.values).copy(), nu=to_host(v.values).copy(),
                      mu_scales=orc.to_f32(to_host(m.scales), DT[scale_dtype]).copy(),
                      nu_scales=orc.to_f32(to_host(v.scales), DT[scale_dtype]).copy())
         else:
@@ -152,6 +152,12 @@ def _adamw8_tree_run(*, scale_dtype, fallback, exact, steps=3, psr=False, clip=N
 @pytest.mark.parametrize("scale_dtype", ["bf16", "f16"])
 def test_adamw8_16_bit_scales_and_f16_params(scale_dtype, exact):
     _adamw8_tree_run(scale_dtype=scale_dtype, fallback="f32", exact=exact)
+
+
+@pytest.mark.parametrize("scale_dtype,exact", [("bf16", True), ("f16", False)])
+@pytest.mark.parametrize("block_size", [128, 1000, 4096])
+def test_adamw8_f16_and_16_bit_scales_other_block_sizes(block_size, scale_dtype, exact):
+    _adamw8_tree_run(scale_dtype=scale_dtype, fallback="f32", exact=exact, block_size=block_size, steps=2)
 
 
 def test_adamw8_f16_fallback_moments_f32_scales():

@@ -150,6 +150,71 @@ def test_noalloc_equals_step_two_calls_second_smaller():
     _run_both(small, 2, 2, _lib.RF_LR | _lib.RF_DECAY_WEAK | _lib.RF_PARAM_SR | _lib.RF_MOMENT_SR, 0.0)
 
 
+@pytest.mark.parametrize("bs", [256, 1000, 4096])
+def test_noalloc_other_block_sizes(bs, monkeypatch):
+    """The tile list beside a generic one, then a short list of the same
+    block size (all in the generic list)."""
+    from rollfast_amd import _lib
+
+    monkeypatch.setitem(globals(), "BS", bs)
+    long = [(1100 * 2048 + 40, "bf16", "bf16", "q"), (5 * bs + 77, "f32", "bf16", "q"), (1000, "bf16", "bf16", "f32"),
+            (4 * bs + 5, "f32", "f32", "f32")]
+    short = [(2 * bs + 3, "bf16", "bf16", "q"), (777, "f32", "f32", "f32")]
+    _run_both(long, 3, 1, _lib.RF_LR | _lib.RF_DECAY_WEAK, 1.0)
+    _run_both(short, 4, 2, _lib.RF_LR | _lib.RF_DECAY_WEAK | _lib.RF_PARAM_SR | _lib.RF_MOMENT_SR, 0.0)
+    _run_both(long, 5, 3, _lib.RF_LR | _lib.RF_PARAM_SR | _lib.RF_MOMENT_SR | _lib.RF_PACKED_BITS, 0.0)
+
+
+def test_noalloc_largest_tree_with_a_tile_list(monkeypatch):
+    """The largest accepted tree that has a tile list and a generic one (the
+    tile list's sentinel is beyond what a tree is charged for) steps as
+    rf_adam8_step does."""
+    import torch
+
+    from rollfast_amd import _lib
+
+    monkeypatch.setitem(globals(), "BS", 256)
+    lib = _lib.lib()
+    hp = _hparams(1, _lib.RF_LR, 0.0)
+    n = _lib.RF_NOALLOC_SCRATCH_BYTES // 120
+    rest = 16
+
+    def tree(seed):
+        gen = torch.Generator(device="cuda")
+        gen.manual_seed(seed)
+        return {"q": _leaf_set([(2100 * 256, "bf16", "bf16", "q")], seed),
+                "arena": [torch.randn(n * rest, generator=gen, device="cuda").abs() for _ in range(4)]}
+
+    def table(t):
+        out = (_lib.Adam8Leaf * n)()
+        out[0] = _table(t["q"])[0]
+        at = [x.data_ptr() for x in t["arena"]]
+        for i in range(1, n):
+            L = out[i]
+            L.param, L.grad, L.mu, L.nu = (a + 4 * rest * i for a in at)
+            L.size = rest
+            L.moment_kind = _lib.RF_MOMENT_F32
+            L.state_index = L.param_index = i
+        return out
+
+    scratch = table(tree(1))
+    lo, hi = 1, n  # lo is accepted, hi refused
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        st = lib.rf_adam8_step_noalloc(scratch, mid, 1, ctypes.byref(hp), _lib.stream_ptr())
+        assert st in (_lib.RF_OK, _lib.RF_ERR_INVALID), lib.rf_last_error()
+        lo, hi = (mid, hi) if st == _lib.RF_OK else (lo, mid)
+    torch.cuda.synchronize()
+    print(f"[no_alloc] largest tree with a tile list: {lo} leaves", flush=True)
+    a, b = tree(2), tree(2)
+    assert lib.rf_adam8_step(table(a), lo, 1, ctypes.byref(hp), _lib.stream_ptr()) == _lib.RF_OK
+    assert lib.rf_adam8_step_noalloc(table(b), lo, 1, ctypes.byref(hp), _lib.stream_ptr()) == _lib.RF_OK
+    torch.cuda.synchronize()
+    _same(a["q"], b["q"], "largest tree")
+    for x, y in zip(a["arena"], b["arena"]):
+        assert torch.equal(x, y)
+
+
 def test_noalloc_refuses_a_tree_beyond_its_scratch():
     import torch
 
