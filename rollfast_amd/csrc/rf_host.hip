@@ -876,15 +876,26 @@ constexpr int64_t short_weight(int64_t bs) { return bs > 512 ? 6 : bs > 128 ? 4 
 // Short lists of full 2048-blocks run in the generic list instead of
 // k_adam8, a workgroup per block: one launch for the tree whatever its
 // dtypes, and four waves on a block's memory latencies and random draws
-// where k_adam8 has one.  Up to 6 blocks per CU for nearest rounding of
-// 16-bit params in the hardware direction, 16 otherwise.  One GPU, a step
-// back to back, k_adam8 and generic launch / merged: 98 blocks f32 21.1 /
-// 7.8 us, bf16 14.7 / 7.6, param SR 44.4 / 9.1, all SR 115.5 / 12.2; 1,568
-// blocks 27.9 / 19.5, 16.9 / 16.1, 46.7 / 24.4, 119.8 / 44.4; 3,141 blocks
-// 36.3 / 31.7, 21.5 / 27.5, 48.6 / 41.7, 125.0 / 77.4; 6,248 blocks 58.3 /
-// 54.3, 38.5 / 48.1, 62.8 / 71.1, 142.7 / 129.4.
-constexpr int64_t MERGE_BLOCKS_PER_CU = 6;
-constexpr int64_t MERGE_BLOCKS_PER_CU_HEAVY = 16;
+// where k_adam8 has one.  How long a list stays short depends on what a
+// block costs a wave (merge_max; blocks per CU): 6 for nearest rounding of
+// 16-bit params and grads in the hardware direction; 12 for their update-only
+// form and param rounding from the packed source, and for nearest rounding
+// with f32 params or grads; 16 for the rest.  Where the generic units would
+// be a launch of their own (no k_adam8 launch to ride along with), the first
+// two are one step further.  One GPU, kernels only, k_adam8 / merged, full
+// blocks alone and (after the semicolon) with a tree's small leaves: bf16
+// nearest 1,536 blocks 16.2 / 14.2 us; 16.7 / 15.4, 2,560 20.1 / 20.9; 20.2 /
+// 22.1.  f16 nearest 2,560 20.2 / 21.6; 27.3 / 22.8, 4,096 21.3 / 30.8; 28.4 /
+// 33.0.  bf16 update-only 2,560 32.0 / 22.4; 32.5 / 32.1, 4,096 35.1 / 32.2;
+// 35.0 / 42.3.  bf16 packed param SR 2,560 34.1 / 26.7; 34.2 / 28.7, 4,096
+// 35.5 / 39.2; 35.6 / 41.8.  f32 nearest 3,141 29.9 / 30.0; 37.4 / 31.0, 4,096
+// 32.9 / 35.5; 40.2 / 37.2.  bf16 exact 4,096 33.9 / 33.4; 34.1 / 35.4, 6,144
+// 42.5 / 47.6.  f32 update-only 4,096 35.6 / 32.6; 45.5 / 37.0.  Jax param SR
+// 4,096 48.1 / 46.3; 48.2 / 47.8, 6,144 60.0 / 66.1.  All SR 4,096 112.4 /
+// 85.8; 124.5 / 81.5.
+constexpr int64_t MERGE_BLOCKS_PER_CU_LIGHT = 6;
+constexpr int64_t MERGE_BLOCKS_PER_CU_MIDDLE = 12;
+constexpr int64_t MERGE_BLOCKS_PER_CU_MAX = 16;
 // Launches of at least this many fast blocks per CU (64 per resident wave
 // at 3 waves per SIMD: far more output than the caches hold) store f32
 // updates and params nontemporally (KHp.upd_nt).
@@ -1895,6 +1906,7 @@ struct rf_adam8_plan {
     std::vector<PlanGroup> groups;
     std::vector<PlanGroup> merged;      // the merged form of a short list (WorkLists::merged), or empty
     int64_t nfast = 0;
+    bool apart = false;                 // as in WorkLists
     bool light = false;                 // light_leaves of its table
     rf_adam8_leaf* d_leaves = nullptr;  // creation-time pointer table
     Seg* d_segs = nullptr;
@@ -1993,6 +2005,7 @@ struct WorkLists {
     std::vector<PlanGroup> groups;   // one launch per list
     std::vector<PlanGroup> merged;   // the launches with the full 2048-blocks in the generic list (short lists only)
     int64_t nfast = 0;               // full 2048-blocks with a k_adam8 instance
+    bool apart = false;              // generic units, and no k_adam8 launch that could take them along
     int64_t units = 0;
     std::vector<Seg> nsegs;          // norm units (NORM_UNIT elements) of the non-empty leaves
     int32_t n_nsegs = 0;
@@ -2008,9 +2021,10 @@ struct WorkLists {
 };
 
 // merge_max: lists of at most this many full 2048-blocks get the merged form
-// too; merged_only: these get no other.
+// too (merge_max_apart: where the generic units launch apart); merged_only:
+// these get no other.
 rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_t apply, int32_t num_cus,
-                           int64_t merge_max, bool merged_only, WorkLists& w)
+                           int64_t merge_max, int64_t merge_max_apart, bool merged_only, WorkLists& w)
 {
     rf_status st = RF_OK;
     std::vector<Seg>* gsegs = w.gsegs;
@@ -2098,12 +2112,13 @@ rf_status build_work_lists(const rf_adam8_leaf* leaves, int32_t n_leaves, int32_
     if (gunits[GEN_LIST] + tile_blocks > INT32_MAX)
         return fail(RF_ERR_UNSUPPORTED, "more than 2^31 - 1 partial or odd-sized quantized blocks in one launch");
     // A second form of the generic list for short lists of full 2048-blocks:
-    // these as leading units too (MERGE_BLOCKS_PER_CU).
+    // these as leading units too (merge_max).
     int64_t nfast = 0;
     for (int c = 0; c <= COMBO_F16; ++c) nfast += gunits[c];
     const int64_t gen_lead = gunits[GEN_LIST];
     w.nfast = nfast;
-    if (nfast > 0 && nfast <= merge_max) {
+    w.apart = gunits[3] == 0 && gunits[GEN_LIST] + gunits[GEN_TAIL] > 0;
+    if (nfast > 0 && nfast <= (w.apart ? merge_max_apart : merge_max)) {
         gsegs[MERGED_LIST] = gsegs[GEN_LIST];
         gunits[MERGED_LIST] = gen_lead;
         for (int c = 0; c <= COMBO_F16; ++c) {
@@ -2247,11 +2262,15 @@ bool light_leaves(const rf_adam8_leaf* leaves, int32_t n)
 }
 
 // Full 2048-blocks up to which a step takes the merged lists.
-int64_t merge_max(const DevState* ds, bool light, uint32_t flags, int32_t apply)
+int64_t merge_max(const DevState* ds, bool light, bool apart, uint32_t flags, int32_t apply)
 {
-    const bool sr = (flags & RF_MOMENT_SR) || ((flags & RF_PARAM_SR) && apply);
-    return ds->num_cus *
-           (light && apply && !sr && !(flags & RF_EXACT) ? MERGE_BLOCKS_PER_CU : MERGE_BLOCKS_PER_CU_HEAVY);
+    const bool psr = (flags & RF_PARAM_SR) && apply, jax_psr = psr && !(flags & RF_PACKED_BITS);
+    int step = (light ? 0 : 1) + (psr || !apply ? 1 : 0) + (apart ? 1 : 0);
+    if ((flags & (RF_MOMENT_SR | RF_EXACT)) || jax_psr) step = 2;
+    const int64_t per_cu = step == 0   ? MERGE_BLOCKS_PER_CU_LIGHT
+                           : step == 1 ? MERGE_BLOCKS_PER_CU_MIDDLE
+                                       : MERGE_BLOCKS_PER_CU_MAX;
+    return ds->num_cus * per_cu;
 }
 
 int64_t step_grid(const DevState* ds, int occ, const PlanGroup& g, int32_t run, int64_t per_wave);
@@ -2320,7 +2339,8 @@ rf_status rf_adam8_plan_create(const rf_adam8_leaf* leaves, int32_t n_leaves, in
     rf_status st = device_state(&ds);
     if (st != RF_OK) return st;
     WorkLists w;
-    st = build_work_lists(leaves, n_leaves, apply, ds->num_cus, MERGE_BLOCKS_PER_CU_HEAVY * ds->num_cus, false, w);
+    const int64_t merge_any = MERGE_BLOCKS_PER_CU_MAX * ds->num_cus;
+    st = build_work_lists(leaves, n_leaves, apply, ds->num_cus, merge_any, merge_any, false, w);
     if (st != RF_OK) return st;
     std::vector<Seg>& segs = w.segs;
     std::vector<Seg>& nsegs = w.nsegs;
@@ -2341,6 +2361,7 @@ rf_status rf_adam8_plan_create(const rf_adam8_leaf* leaves, int32_t n_leaves, in
     p->groups = w.groups;
     p->merged = w.merged;
     p->nfast = w.nfast;
+    p->apart = w.apart;
     p->light = light_leaves(leaves, n_leaves);
     p->cover = bits_cover(leaves, n_leaves);
     p->shape.assign(leaves, leaves + n_leaves);
@@ -2611,7 +2632,7 @@ rf_status plan_launch(const rf_adam8_plan* plan, const rf_adam8_leaf* d_leaves, 
     // launch instead of two.
     const PlanGroup* gen = nullptr;
     const PlanGroup* carrier = nullptr;
-    const bool merged = !plan->merged.empty() && plan->nfast <= merge_max(ds, plan->light, f, plan->apply);
+    const bool merged = !plan->merged.empty() && plan->nfast <= merge_max(ds, plan->light, plan->apart, f, plan->apply);
     const std::vector<PlanGroup>& groups = merged ? plan->merged : plan->groups;
     find_carrier(groups, msr, &gen, &carrier);
     k.gsegs = nullptr;
@@ -2871,8 +2892,9 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     std::lock_guard<std::mutex> order(ds->noalloc_mu);
     // Host-side lists in per-thread buffers that keep their capacity.
     thread_local WorkLists w;
-    st = build_work_lists(leaves, n_leaves, apply, ds->num_cus,
-                          merge_max(ds, light_leaves(leaves, n_leaves), hp->flags, apply), true, w);
+    const bool light = light_leaves(leaves, n_leaves);
+    st = build_work_lists(leaves, n_leaves, apply, ds->num_cus, merge_max(ds, light, false, hp->flags, apply),
+                          merge_max(ds, light, true, hp->flags, apply), true, w);
     if (st != RF_OK) return st;
 
     // Scratch layout: what the host stages (leaf table, group table, step and
@@ -2921,7 +2943,8 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     plan.groups.swap(w.groups);  // lent for the launch, then handed back with their capacity
     plan.merged.swap(w.merged);
     plan.nfast = w.nfast;
-    plan.light = light_leaves(leaves, n_leaves);
+    plan.apart = w.apart;
+    plan.light = light;
     plan.d_leaves = (rf_adam8_leaf*)base;
     plan.d_segs = (Seg*)(base + o_segs);
     plan.d_nsegs = (Seg*)(base + o_nsegs);
