@@ -230,10 +230,12 @@ RF_API rf_status rf_adam8_plan_run_leaves(rf_adam8_plan* plan, const rf_adam8_le
  * (an empty run never writes finite_host). */
 RF_API rf_status rf_adam8_plan_wait_prepass(const rf_adam8_plan* plan);
 
-/* Number of step-kernel launches, leaves and work units of a plan.  A plan
- * with full blocks of bf16 params and grads launches its generic units
- * (partial blocks, small leaves) inside that launch: one launch for such a
- * tree, one more per other (param, grad) dtype pair with full blocks. */
+/* Number of step-kernel launches (of a run without rounding or direction
+ * flags on this device), leaves and work units of a plan.  Full blocks of
+ * 2048 are a launch per (param, grad) dtype pair, which with bf16 params and
+ * grads takes the generic units (partial blocks, small leaves) along; a tree
+ * with few of them runs them among its generic units, one launch in all.
+ * Long lists of other block sizes are a launch of their own. */
 RF_API rf_status rf_adam8_plan_info(const rf_adam8_plan* plan, int64_t* launches, int64_t* leaves,
                              int64_t* units);
 

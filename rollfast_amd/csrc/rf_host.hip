@@ -1906,6 +1906,7 @@ struct rf_adam8_plan {
     std::vector<PlanGroup> groups;
     std::vector<PlanGroup> merged;      // the merged form of a short list (WorkLists::merged), or empty
     int64_t nfast = 0;
+    int32_t num_cus = 0;                // of its device
     bool apart = false;                 // as in WorkLists
     bool light = false;                 // light_leaves of its table
     rf_adam8_leaf* d_leaves = nullptr;  // creation-time pointer table
@@ -2262,7 +2263,7 @@ bool light_leaves(const rf_adam8_leaf* leaves, int32_t n)
 }
 
 // Full 2048-blocks up to which a step takes the merged lists.
-int64_t merge_max(const DevState* ds, bool light, bool apart, uint32_t flags, int32_t apply)
+int64_t merge_max(int64_t num_cus, bool light, bool apart, uint32_t flags, int32_t apply)
 {
     const bool psr = (flags & RF_PARAM_SR) && apply, jax_psr = psr && !(flags & RF_PACKED_BITS);
     int step = (light ? 0 : 1) + (psr || !apply ? 1 : 0) + (apart ? 1 : 0);
@@ -2270,7 +2271,16 @@ int64_t merge_max(const DevState* ds, bool light, bool apart, uint32_t flags, in
     const int64_t per_cu = step == 0   ? MERGE_BLOCKS_PER_CU_LIGHT
                            : step == 1 ? MERGE_BLOCKS_PER_CU_MIDDLE
                                        : MERGE_BLOCKS_PER_CU_MAX;
-    return ds->num_cus * per_cu;
+    return num_cus * per_cu;
+}
+
+// The launches of a run with `flags`: the merged form of a list short enough
+// for them.
+const std::vector<PlanGroup>& run_groups(const rf_adam8_plan* plan, uint32_t flags)
+{
+    const bool merged =
+        !plan->merged.empty() && plan->nfast <= merge_max(plan->num_cus, plan->light, plan->apart, flags, plan->apply);
+    return merged ? plan->merged : plan->groups;
 }
 
 int64_t step_grid(const DevState* ds, int occ, const PlanGroup& g, int32_t run, int64_t per_wave);
@@ -2361,6 +2371,7 @@ rf_status rf_adam8_plan_create(const rf_adam8_leaf* leaves, int32_t n_leaves, in
     p->groups = w.groups;
     p->merged = w.merged;
     p->nfast = w.nfast;
+    p->num_cus = ds->num_cus;
     p->apart = w.apart;
     p->light = light_leaves(leaves, n_leaves);
     p->cover = bits_cover(leaves, n_leaves);
@@ -2406,11 +2417,10 @@ rf_status rf_adam8_plan_info(const rf_adam8_plan* plan, int64_t* launches, int64
 {
     if (!plan) return fail(RF_ERR_INVALID, "null plan");
     if (launches) {
-        // the generic list rides along with a bf16/bf16 fast launch (plan_launch)
+        const std::vector<PlanGroup>& groups = run_groups(plan, 0);
         const PlanGroup *gen = nullptr, *carrier = nullptr;
-        find_carrier(plan->groups, false, &gen, &carrier);
-        *launches = (int64_t)plan->groups.size() - (carrier ? 1 : 0);
-        if (!plan->merged.empty()) *launches = std::min(*launches, (int64_t)plan->merged.size());
+        find_carrier(groups, false, &gen, &carrier);
+        *launches = (int64_t)groups.size() - (carrier ? 1 : 0);
     }
     if (leaves) *leaves = plan->n_leaves;
     if (units) *units = plan->total_units;
@@ -2632,8 +2642,7 @@ rf_status plan_launch(const rf_adam8_plan* plan, const rf_adam8_leaf* d_leaves, 
     // launch instead of two.
     const PlanGroup* gen = nullptr;
     const PlanGroup* carrier = nullptr;
-    const bool merged = !plan->merged.empty() && plan->nfast <= merge_max(ds, plan->light, plan->apart, f, plan->apply);
-    const std::vector<PlanGroup>& groups = merged ? plan->merged : plan->groups;
+    const std::vector<PlanGroup>& groups = run_groups(plan, f);
     find_carrier(groups, msr, &gen, &carrier);
     k.gsegs = nullptr;
     k.gunits = 0;
@@ -2893,8 +2902,8 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     // Host-side lists in per-thread buffers that keep their capacity.
     thread_local WorkLists w;
     const bool light = light_leaves(leaves, n_leaves);
-    st = build_work_lists(leaves, n_leaves, apply, ds->num_cus, merge_max(ds, light, false, hp->flags, apply),
-                          merge_max(ds, light, true, hp->flags, apply), true, w);
+    st = build_work_lists(leaves, n_leaves, apply, ds->num_cus, merge_max(ds->num_cus, light, false, hp->flags, apply),
+                          merge_max(ds->num_cus, light, true, hp->flags, apply), true, w);
     if (st != RF_OK) return st;
 
     // Scratch layout: what the host stages (leaf table, group table, step and
@@ -2943,6 +2952,7 @@ rf_status rf_adam8_step_noalloc(const rf_adam8_leaf* leaves, int32_t n_leaves, i
     plan.groups.swap(w.groups);  // lent for the launch, then handed back with their capacity
     plan.merged.swap(w.merged);
     plan.nfast = w.nfast;
+    plan.num_cus = ds->num_cus;
     plan.apart = w.apart;
     plan.light = light;
     plan.d_leaves = (rf_adam8_leaf*)base;

@@ -92,6 +92,41 @@ def test_one_shot_step_through_the_abi():
     _compare(bufs, host)
 
 
+@pytest.mark.parametrize("blocks,launches", [(1000, 1), (1000 + 2 * 768, 2)])
+def test_plan_info_counts_the_launches_of_a_run(blocks, launches):
+    """bf16 and f16 leaves of full blocks: one launch while the tree is short
+    enough for a nearest-rounding run to merge them (6 blocks per CU), two
+    beyond, also where other flags would still merge them."""
+    import torch
+
+    from rollfast_amd import _lib
+
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n = blocks * cus // 256 // 2 * 2048
+    assert (2 * n // 2048 <= 6 * cus) == (launches == 1) and 2 * n // 2048 <= 12 * cus
+    table = (_lib.Adam8Leaf * 2)()
+    keep = []
+    for i, dt in enumerate((torch.bfloat16, torch.float16)):
+        p, g = torch.zeros(n, dtype=dt, device="cuda"), torch.zeros(n, dtype=dt, device="cuda")
+        codes = torch.zeros(2 * n, dtype=torch.uint8, device="cuda")
+        scales = torch.ones(2 * n // 2048, device="cuda")
+        keep += [p, g, codes, scales]
+        L = table[i]
+        L.param, L.grad, L.mu, L.nu = p.data_ptr(), g.data_ptr(), codes.data_ptr(), codes.data_ptr() + n
+        L.mu_scales, L.nu_scales = scales.data_ptr(), scales.data_ptr() + 4 * (n // 2048)
+        L.size, L.block_size, L.moment_kind = n, 2048, _lib.RF_MOMENT_QUANTIZED
+        L.param_dtype = L.grad_dtype = _lib.RF_BF16 if dt == torch.bfloat16 else _lib.RF_F16
+        L.state_index = L.param_index = i
+    plan, got = ctypes.c_void_p(), ctypes.c_int64()
+    lib = _lib.lib()
+    assert lib.rf_adam8_plan_create(table, 2, 1, ctypes.byref(plan)) == _lib.RF_OK
+    try:
+        assert lib.rf_adam8_plan_info(plan, ctypes.byref(got), None, None) == _lib.RF_OK
+        assert got.value == launches
+    finally:
+        assert lib.rf_adam8_plan_destroy(plan) == _lib.RF_OK
+
+
 def test_plan_run_on_creation_table_and_info():
     import torch
 
