@@ -279,6 +279,17 @@ __global__ __launch_bounds__(WG) void k_quantize(int32_t quantizer, const void* 
 // Multiples of 8 that no other kernel takes: one wave per block in two passes
 // of vector accesses, the second of which finds the block in L2.  2^26 f32
 // in blocks of 4096 and 1000: 89 and 95 us; element by element 202 and 205.
+// A row of 512 elements takes its eight codes per lane whether the block
+// fills it or not, and stochastic rounding draws them one after the other:
+// a block's last part-row goes an element per lane at a time up to VEC_TAIL
+// elements (VEC_TAIL_SR with the draws).  2^24 f32, all vectors / with that
+// rule: blocks of 520 33 / 27 us, of 1032 25 / 22 and with draws 117 / 85.
+constexpr int64_t VEC_TAIL = 64;
+constexpr int64_t VEC_TAIL_SR = 360;
+// Blocks at most this long are not worth a row at all (rf_blockwise_quantize).
+constexpr int64_t VEC_MIN = 192;
+constexpr int64_t VEC_MIN_INT8 = 256;
+constexpr int64_t VEC_TAIL_SHORT_SR = 448;
 __global__ __launch_bounds__(WG) void k_quantize_vec(QuantArgs q, int64_t bs, const uint4* __restrict__ tables)
 {
     __shared__ __attribute__((aligned(16))) uint8_t lds[TABLE_BYTES];
@@ -289,7 +300,8 @@ __global__ __launch_bounds__(WG) void k_quantize_vec(QuantArgs q, int64_t bs, co
     for (int64_t b = wave; b < q.nblocks; b += nwaves) {
         const int64_t base = b * bs;
         const int64_t nvalid = max((int64_t)0, min(bs, q.size - base));
-        const int64_t nvec = nvalid / 8 * 8;
+        const int64_t whole = nvalid / 512 * 512;
+        const int64_t nvec = nvalid - whole > (q.sr ? VEC_TAIL_SR : VEC_TAIL) ? nvalid / 8 * 8 : whole;
         uint32_t am = 0;
 #pragma unroll 4
         for (int64_t j = lane * 8; j < nvec; j += WAVE * 8) {
@@ -2992,10 +3004,18 @@ rf_status rf_blockwise_quantize(int32_t quantizer, const void* x, int32_t x_dtyp
     unsigned grid = 1;
     // Aligned buffers in blocks of other multiples of 8 than 2048: powers of
     // two up to a wave's tile take the tile kernel, the rest the two vector
-    // passes; everything else k_quantize.
-    if (aligned(x, 16) && aligned(values, 8) && block_size % 8 == 0 && block_size != FAST_BS) {
+    // passes; everything else k_quantize, and so do short blocks that are no
+    // power of two, of which a row of vectors would be mostly empty.  2^24
+    // f32, k_quantize / two vector passes: blocks of 24 175 / 389 us, 136 64 /
+    // 74, 264 51 / 40; int8 200 54 / 61, 264 51 / 47; with draws 24 259 /
+    // 1,420, 392 92 / 100, 456 95 / 90, 776 85 / 93, 904 91 / 85.
+    const bool tiled = block_size <= TILE_SPAN && (block_size & (block_size - 1)) == 0;
+    const bool short_rows =
+        !tiled && (sr ? block_size < 1024 && block_size % 512 <= (block_size < 512 ? VEC_TAIL_SHORT_SR : VEC_TAIL_SR)
+                      : block_size <= (quantizer == RF_Q_SYMMETRIC_INT8 ? VEC_MIN_INT8 : VEC_MIN));
+    if (aligned(x, 16) && aligned(values, 8) && block_size % 8 == 0 && block_size != FAST_BS && !short_rows) {
         const QuantArgs q{x, (uint8_t*)values, scales, bits, size, nb, key0, key1, quantizer, x_dtype, scale_dtype, sr};
-        if (block_size <= TILE_SPAN && (block_size & (block_size - 1)) == 0) {
+        if (tiled) {
             const int32_t lg = 31 - __builtin_clz((unsigned)block_size);
             st = worklist_grid((const void*)&k_quantize_tile, ds, (nb * block_size + TILE_SPAN - 1) / TILE_SPAN, &grid,
                                8);

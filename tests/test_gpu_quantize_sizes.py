@@ -1,6 +1,7 @@
 """quantize_blocks over the block sizes of its layouts (powers of two up to
 1024 in 1024-element tiles; 2048 in registers; other sizes a wave per block,
-by vectors where the size is a multiple of 8) and dequantize_blocks over its
+by vectors where the size is a multiple of 8 and no short one, a short last
+row aside) and dequantize_blocks over its
 own (powers of two, other multiples of 4, odd sizes), against the CPU oracle
 bit for bit, and on an unaligned input."""
 
@@ -15,7 +16,8 @@ from tests.test_gpu_kernels import QUANTIZERS, _edge_values
 
 pytestmark = pytest.mark.gpu
 
-BLOCK_SIZES = [3, 4, 8, 12, 16, 24, 32, 64, 128, 256, 512, 1000, 1024, 1028, 2040, 2048, 4096, 5000, 8192]
+BLOCK_SIZES = [3, 4, 8, 12, 16, 24, 32, 64, 128, 192, 200, 256, 264, 448, 456, 512, 520, 576, 584, 872, 880, 1000, 1024,
+               1028, 1032, 2040, 2048, 4096, 5000, 8192]
 
 
 def _check(x, dtype, bs, quantizer, sr, offset=0):
