@@ -752,37 +752,11 @@ __device__ __forceinline__ float acc_op(int32_t mode, int32_t cdt, float g, floa
 }
 
 // Four consecutive values of an f32, bf16 or f16 array (8-byte or, f32,
-// 16-byte aligned).
-__device__ __forceinline__ void ld4_dt(const void* base, int32_t dtype, int64_t e0, float (&x)[4])
-{
-    if (dtype == RF_F32) {
-        const float4 v = *(const float4*)((const float*)base + e0);
-        x[0] = v.x;
-        x[1] = v.y;
-        x[2] = v.z;
-        x[3] = v.w;
-    } else {
-        unpack4_h16(*(const nt_u32x2*)((const uint16_t*)base + e0), dtype, x);
-    }
-}
-
-// The same, nontemporal.
+// 16-byte aligned), nontemporal.
 __device__ __forceinline__ void ld4_dt_nt(const void* base, int32_t dtype, int64_t e0, float (&x)[4])
 {
     if (dtype == RF_F32) ld4_f32_nt(base, e0, x);
     else unpack4_h16(ld4_h16_nt(base, e0), dtype, x);
-}
-
-__device__ __forceinline__ void st4_dt(void* base, int32_t dtype, int64_t e0, const float (&x)[4])
-{
-    if (dtype == RF_F32) {
-        *(float4*)((float*)base + e0) = make_float4(x[0], x[1], x[2], x[3]);
-    } else {
-        const bool f16 = dtype == RF_F16;
-        *(uint2*)((uint16_t*)base + e0) =
-            make_uint2(f16 ? pack_f16x2_rne(x[0], x[1]) : pack_bf16x2_rne(x[0], x[1]),
-                       f16 ? pack_f16x2_rne(x[2], x[3]) : pack_bf16x2_rne(x[2], x[3]));
-    }
 }
 
 __global__ __launch_bounds__(WG) void k_accumulate(const rf_accum_leaf* __restrict__ leaves,
@@ -815,10 +789,36 @@ __global__ __launch_bounds__(WG) void k_accumulate(const rf_accum_leaf* __restri
         // step: 1.496 -> 1.459 ms; two or four such groups in flight 1.467
         // and 1.554, and nontemporal accumulators 1.755 (a micro-step finds
         // part of what the last one wrote in the memory-side cache).
-        const int64_t v_end = vec ? e_begin + ((e_end - e_begin) / 4) * 4 : e_begin;
-        for (int64_t e0 = e_begin + lane * 4; e0 < v_end; e0 += WAVE * 4) {
+        // 16-bit accumulators take eight, for the same reason: 64 M bf16
+        // elements, a window of four bf16 micro-steps with its step, 476 us,
+        // four per lane 585.
+        const int64_t w = L.acc_dtype == RF_F32 ? 4 : 8;
+        const int64_t v_end = vec ? e_begin + (e_end - e_begin) / w * w : e_begin;
+        for (int64_t e0 = e_begin + lane * 8; w == 8 && e0 < v_end; e0 += WAVE * 8) {
+            float g[8], a[8];
+            load8_dt(L.acc, L.acc_dtype, e0, a);
+            if (mode == RF_ACC_ZERO) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t) a[t] = 0.0f * a[t];
+            } else {
+                load8_dt(L.grad, L.grad_dtype, e0, g);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) a[t] = acc_op(mode, cdt, g[t], a[t], div);
+            }
+            uint32_t h[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                h[t] = L.acc_dtype == RF_F16 ? pack_f16x2_rne(a[2 * t], a[2 * t + 1])
+                                             : pack_bf16x2_rne(a[2 * t], a[2 * t + 1]);
+            *(uint4*)((uint16_t*)L.acc + e0) = make_uint4(h[0], h[1], h[2], h[3]);
+        }
+        for (int64_t e0 = e_begin + lane * 4; w == 4 && e0 < v_end; e0 += WAVE * 4) {
             float g[4], a[4];
-            ld4_dt(L.acc, L.acc_dtype, e0, a);
+            const float4 av = *(const float4*)((const float*)L.acc + e0);
+            a[0] = av.x;
+            a[1] = av.y;
+            a[2] = av.z;
+            a[3] = av.w;
             if (mode == RF_ACC_ZERO) {
 #pragma unroll
                 for (int t = 0; t < 4; ++t) a[t] = 0.0f * a[t];
@@ -827,7 +827,7 @@ __global__ __launch_bounds__(WG) void k_accumulate(const rf_accum_leaf* __restri
 #pragma unroll
                 for (int t = 0; t < 4; ++t) a[t] = acc_op(mode, cdt, g[t], a[t], div);
             }
-            st4_dt(L.acc, L.acc_dtype, e0, a);
+            *(float4*)((float*)L.acc + e0) = make_float4(a[0], a[1], a[2], a[3]);
         }
         for (int64_t e = v_end + lane; e < e_end; e += WAVE) {
             const float a = load1(L.acc, L.acc_dtype, e);
