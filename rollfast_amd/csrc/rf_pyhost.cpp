@@ -546,6 +546,22 @@ int rf_dtype(at::ScalarType t)
     return t == at::kFloat ? RF_F32 : t == at::kBFloat16 ? RF_BF16 : t == at::kHalf ? RF_F16 : -1;
 }
 
+bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w);
+
+// A container's child: containers nested beyond Python's recursion limit are
+// left to the Python walk, whose RecursionError they get.
+bool accum_child(PyObject* g, PyObject* a, AccumWalk& w)
+{
+    if (Py_EnterRecursiveCall(" in a tree walk")) {
+        PyErr_Clear();
+        return false;
+    }
+    struct Leave {
+        ~Leave() { Py_LeaveRecursiveCall(); }
+    } leave;
+    return accum_walk(g, a, w);
+}
+
 bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w)
 {
     if (is_aux(a)) return w.reset || is_grad_leaf(g);
@@ -581,7 +597,7 @@ bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w)
             PyObject* ca = PyDict_GetItemWithError(a, key);
             PyObject* cg = w.reset ? Py_None : PyDict_GetItemWithError(g, key);
             try {
-                ok = ca && cg && accum_walk(cg, ca, w);
+                ok = ca && cg && accum_child(cg, ca, w);
             } catch (const std::exception&) {
                 ok = false;
             }
@@ -596,7 +612,7 @@ bool accum_walk(PyObject* g, PyObject* a, AccumWalk& w)
     if (!w.reset && ((is_list ? !PyList_CheckExact(g) : !PyTuple_CheckExact(g)) || PySequence_Fast_GET_SIZE(g) != n))
         return false;
     for (Py_ssize_t k = 0; k < n; ++k)
-        if (!accum_walk(w.reset ? Py_None : PySequence_Fast_GET_ITEM(g, k), PySequence_Fast_GET_ITEM(a, k), w))
+        if (!accum_child(w.reset ? Py_None : PySequence_Fast_GET_ITEM(g, k), PySequence_Fast_GET_ITEM(a, k), w))
             return false;
     return true;
 }

@@ -6,6 +6,9 @@ to refuse host tensors instead of falling back to a CPU path."""
 from __future__ import annotations
 
 import inspect
+import os
+import subprocess
+import sys
 from typing import NamedTuple
 
 import numpy as np
@@ -439,6 +442,26 @@ def test_native_accumulation_walk_leaves_subclasses_to_python():
     with pytest.raises((RuntimeError, ValueError, AssertionError)):  # no GPU, or the null pointer refused
         ms.update._accumulate(Inner(), Inner(), _lib.RF_ACC_SUM, 0)
     assert "data_ptr" in asked
+
+
+def test_native_accumulation_walk_of_deeply_nested_containers():
+    """Containers nested beyond the recursion limit get the Python walk's
+    RecursionError (a native recursion without a limit overflows the C stack,
+    so in a process of its own)."""
+    code = ("from rollfast_amd import _lib\n"
+            "import rollfast_amd as rf\n"
+            "for wrap in (lambda x: [x], lambda x: {'w': x}):\n"
+            "    tree = None\n"
+            "    for _ in range(300000):\n"
+            "        tree = wrap(tree)\n"
+            "    assert _lib.pyhost().accum_rows(None, tree) is None\n"
+            "    try:\n"
+            "        rf.MultiSteps(rf.adamw8(1e-3), 2).update._accumulate(None, tree, _lib.RF_ACC_ZERO, 0)\n"
+            "    except RecursionError:\n"
+            "        print('refused')\n")
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100,
+                          cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert done.returncode == 0 and done.stdout.split() == ["refused", "refused"], (done.returncode, done.stderr)
 
 
 def test_bias_correction_ignores_the_callers_error_state():
