@@ -11,11 +11,11 @@
 // so nothing is read twice.  Only the absmax reduction and the scales differ
 // by block size:
 //
-//   KIND_QTILE  block sizes 8, 16, .. 1024 (powers of two): a span holds
-//               whole blocks, a block being 1 to 64 lanes of a chunk, or the
-//               two chunks; one scale per lane and chunk.
-//   KIND_QWAVE  other multiples of 8 below 1024: a wave per block, its last
-//               lanes idle.
+//   KIND_QTILE  block sizes 8, 16, .. 512 (powers of two): a span holds
+//               whole blocks, a block being 1 to 64 lanes of a chunk; one
+//               scale per lane and chunk.
+//   KIND_QWAVE  1024, and other multiples of 8 below it: a wave per block,
+//               its last lanes idle.
 //   KIND_QTEAM  multiples of 8 from 1032 to 4096: a workgroup per block, a
 //               quarter of it per wave, the absmax meeting in LDS.  In the
 //               generic list: blocks of 2048, one chunk per wave.
@@ -322,6 +322,103 @@ __device__ __forceinline__ uint2 tile_code8_stream(const UnitCtx& c, const uint3
     return make_uint2(pack4_u8(cc[0], cc[1], cc[2], cc[3]), pack4_u8(cc[4], cc[5], cc[6], cc[7]));
 }
 
+// One moment's codes by the literal search (code_literal), whatever the
+// scale: the eight searches advance together, so a step of theirs is one LDS
+// round trip; the draws are made one at a time, which keeps this rare path
+// short.
+template <bool MSR, bool SECOND>
+__device__ __forceinline__ uint2 tile_code8_literal(const UnitCtx& c, const rf_adam8_leaf& L, int64_t e0,
+                                                    const float (&x)[8], float s)
+{
+    const float* cb = (const float*)(c.lds + (SECOND ? L_CBU : L_CBS));
+    uint32_t bits[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if constexpr (MSR) {
+#pragma unroll 1
+        for (int t = 0; t < 8; ++t) {
+#pragma unroll
+            for (int k = 0; k < 7; ++k) bits[k] = bits[k + 1];
+            bits[7] = SECOND ? nu_bits1(c, L, e0 + t) : mu_bits1(c, L, e0 + t);
+        }
+    }
+    const float lo = cb[0], hi = cb[255];
+    float n[8];
+    uint32_t pos[8];
+    bool nan[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        n[t] = x[t] / s;  // IEEE division
+        nan[t] = n[t] != n[t];
+        n[t] = n[t] < lo ? lo : n[t];
+        n[t] = n[t] > hi ? hi : n[t];
+        pos[t] = 0;
+    }
+#pragma unroll 1
+    for (uint32_t step = 128; step >= 1; step >>= 1) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) pos[t] += cb[pos[t] + step - 1] < n[t] ? step : 0u;
+    }
+    uint32_t code[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const uint32_t ui = pos[t], li = ui > 0 ? ui - 1 : 0;
+        const float lv = cb[li], uv = cb[ui];
+        bool upper;
+        if constexpr (MSR) {
+            const float den = uv - lv;
+            float p = den > 0.0f ? (n[t] - lv) / den : 0.0f;
+            p = p < 0.0f ? 0.0f : (p > 1.0f ? 1.0f : p);
+            upper = uniform_from_bits(bits[t]) < p;
+        } else {
+            upper = fabsf(uv - n[t]) < fabsf(n[t] - lv);
+        }
+        code[t] = nan[t] ? 254u : upper ? ui : li;
+    }
+    return make_uint2(pack4_u8(code[0], code[1], code[2], code[3]), pack4_u8(code[4], code[5], code[6], code[7]));
+}
+
+// Each block's absmax bits, from the lanes' own, in all of the block's lanes.
+// `team`: the workgroup's four waves hold the parts of one block, whose bits
+// meet in `red`; called by every wave.
+template <bool WHOLE, int J>
+__device__ __forceinline__ void tile_block_max(uint32_t (&am)[J], uint32_t (&av)[J], int32_t lg, bool team,
+                                               uint32_t* red)
+{
+    if (lg < 10) {
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            am[j] = tile_max(am[j], lg);
+            av[j] = tile_max(av[j], lg);
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 1; j < J; ++j) {
+        am[0] = max(am[0], am[j]);
+        av[0] = max(av[0], av[j]);
+    }
+    am[0] = wave_max_u32(am[0]);
+    av[0] = wave_max_u32(av[0]);
+    if (!WHOLE && team) {
+        const int w = (int)uniform_u32(threadIdx.x / WAVE);
+        if ((threadIdx.x & (WAVE - 1)) == 0) {
+            red[2 * w] = am[0];
+            red[2 * w + 1] = av[0];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < WAVES_PER_WG; ++k) {
+            am[0] = max(am[0], red[2 * k]);
+            av[0] = max(av[0], red[2 * k + 1]);
+        }
+        __syncthreads();  // red is free again
+    }
+#pragma unroll
+    for (int j = 1; j < J; ++j) {
+        am[j] = am[0];
+        av[j] = av[0];
+    }
+}
+
 // The direction of eight elements, Nesterov's by a uniform branch.
 template <bool EXACT>
 __device__ __forceinline__ void tile_direction8(const KHp& h, bool nest, const float (&m)[8], const float (&v)[8],
@@ -343,12 +440,16 @@ __device__ __forceinline__ void tile_direction8(const KHp& h, bool nest, const f
 // is requantized (len 0: none).  WHOLE: the span is TILE_SPAN elements of
 // the leaf, and so is `next`.  That instance has no masks: every path through
 // it issues the same number of memory operations, so the compiler's waits
-// for a chunk's loads leave the later stores in flight.
+// for a chunk's loads leave the later stores in flight.  Nor has it the
+// literal search: it returns false for a span with a tiny, infinite or NaN
+// scale, its params stored, codes and scales as they were, which the caller
+// gives to the other instance with `codes_only` (true: the params or updates
+// are not written again).
 // J: the span's chunks at most.
 template <int32_t DT, bool APPLY, bool MSR, bool PSR, bool EXACT, bool WHOLE, int J>
-__device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf& L, const KHp& h, bool nest, bool team,
+__device__ __forceinline__ bool unit_tile(const UnitCtx& c, const rf_adam8_leaf& L, const KHp& h, bool nest, bool team,
                                           const TileSpan& sp, TileSlot (&sl)[2], bool have0, const TileSpan& next,
-                                          uint32_t* red)
+                                          uint32_t* red, bool codes_only = false)
 {
     const int lane = threadIdx.x & (WAVE - 1);
     const int32_t pdt = DT == DT_ANY ? L.param_dtype : DT, gdt = DT == DT_ANY ? L.grad_dtype : DT;
@@ -451,7 +552,7 @@ __device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf&
                 }
             }
         }
-        if (nv > 0) {
+        if (nv > 0 && (WHOLE || !codes_only)) {
             if constexpr (!APPLY) {
                 tile_store8_f32(L.updates, sp.base, eo, nv, u);
             } else if (pdt == RF_F32) {
@@ -481,60 +582,57 @@ __device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf&
         }
     }
 
-    // Each block's absmax in all of its lanes.
+    // Each block's absmax in all of its lanes.  Old scales that are not
+    // finite make the block slow (below) wherever it is.
     const int32_t lg = sp.lg;
-    if (lg >= 10) {
+    if (odd != 0) {
 #pragma unroll
-        for (int j = 1; j < J; ++j) {
-            am[0] = max(am[0], am[j]);
-            av[0] = max(av[0], av[j]);
-        }
-        am[0] = wave_max_u32(am[0]);
-        av[0] = wave_max_u32(av[0]);
-        if (!WHOLE && team) {
-            const int w = (int)uniform_u32(threadIdx.x / WAVE);
-            // (every part that is not empty sees the block's old scales: a part's `odd` makes the block slow in all)
-            if (lane == 0) {
-                red[2 * w] = am[0];
-                red[2 * w + 1] = odd ? 0x7FFFFFFFu : av[0];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int k = 0; k < WAVES_PER_WG; ++k) {
-                am[0] = max(am[0], red[2 * k]);
-                av[0] = max(av[0], red[2 * k + 1]);
-            }
-            __syncthreads();  // red is free for the workgroup's next block
-        }
-#pragma unroll
-        for (int j = 1; j < J; ++j) {
-            am[j] = am[0];
-            av[j] = av[0];
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            am[j] = tile_max(am[j], lg);
-            av[j] = tile_max(av[j], lg);
-        }
+        for (int j = 0; j < J; ++j) av[j] = 0x7FFFFFFFu;
     }
+    tile_block_max<WHOLE, J>(am, av, lg, team, red);
     float sm[J], sv[J];
-    uint64_t slow = odd;
+    uint64_t slow = 0;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
         sm[j] = scale_from_absmax_bits(am[j]);
         sv[j] = scale_from_absmax_bits(av[j]);
         slow |= __builtin_amdgcn_ballot_w64(!(block_is_fast(am[j], sm[j]) && block_is_fast(av[j], sv[j])));
     }
-    if (__builtin_expect(slow != 0, 0)) {
-        // A block of the span with a tiny, infinite or NaN scale: the span's
-        // blocks are recomputed from their old codes and scales, which are
-        // still in place, and coded literally where needed.
-        const int64_t nblk = !WHOLE && team ? (uniform_u32(threadIdx.x / WAVE) == 0 ? 1 : 0)
-                             : lg >= 10     ? 1
-                                            : (int64_t)(sp.len >> lg);
-        for (int64_t b = 0; b < nblk; ++b) requant_literal<MSR, 1>(c, L, sp.blk0 + b, h);
-        return;
+    if constexpr (WHOLE) {
+        if (__builtin_expect(slow != 0, 0)) return false;
+    } else if (__builtin_expect(slow != 0, 0)) {
+        // A block of the span with a tiny, infinite or NaN scale (in a team:
+        // the workgroup's block, so that every wave is here): the span's
+        // moments, still in registers, are coded by the literal search under
+        // the reference's NaN-propagating absmax (adam8.py:142).  2^24 bf16
+        // elements, nearest, one block in 16 of that kind, one GPU: blocks of
+        // 8 116 us, of 256 70, of 4096 96; 1,139, 88 and 503 with one wave
+        // recomputing the span's blocks one after the other.  The same code
+        // in the WHOLE instance too cost spans without such blocks 4 %.
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            am[j] = av[j] = 0;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                am[j] = max(am[j], __float_as_uint(m[j][t]) & 0x7FFFFFFFu);
+                av[j] = max(av[j], __float_as_uint(v[j][t]));
+            }
+        }
+        tile_block_max<WHOLE, J>(am, av, lg, team, red);
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const int32_t eo = j * 512 + lane * 8;
+            if (eo >= sp.len) continue;
+            const float s1 = scale_from_absmax_bits(am[j]), s2 = scale_from_absmax_bits(av[j]);
+            st_nt(tile_ptr<uint2>(L.mu, sp.base, 1, eo), tile_code8_literal<MSR, false>(c, L, sp.base + eo, m[j], s1));
+            st_nt(tile_ptr<uint2>(L.nu, sp.base, 1, eo), tile_code8_literal<MSR, true>(c, L, sp.base + eo, v[j], s2));
+            if (!team || threadIdx.x < WAVE) {
+                const int64_t blk = sp.blk0 + (eo >> lg);
+                store_scale(L.mu_scales, L.flags, blk, s1);
+                store_scale(L.nu_scales, L.flags, blk, s2);
+            }
+        }
+        return true;
     }
 #pragma unroll
     for (int j = 0; j < J; ++j) {
@@ -564,6 +662,7 @@ __device__ __forceinline__ void unit_tile(const UnitCtx& c, const rf_adam8_leaf&
             }
         }
     }
+    return true;
 }
 
 // The part of element range [lo, hi) of the leaf's code array as a span.

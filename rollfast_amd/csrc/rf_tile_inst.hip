@@ -107,11 +107,12 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(RF_TILE_WAVE
                 next = span(nlead + un);
                 if (next.rem < TILE_SPAN) next.len = 0;
             }
-            if (whole)
-                unit_tile<DT, APPLY, MSR, PSR, EXACT, true, TJ>(c, L, hl, nest, false, sp, sl, have0, next, red);
-            else
-                unit_tile<DT, APPLY, MSR, PSR, EXACT, false, TJ>(c, L, hl, nest, false, sp, sl, false, next, red);
-            have0 = next.len > 0;
+            const bool done =
+                whole && unit_tile<DT, APPLY, MSR, PSR, EXACT, true, TJ>(c, L, hl, nest, false, sp, sl, have0, next, red);
+            if (!done)  // a short span, or the codes of one with a slow block (the next one's chunk is loaded anew)
+                unit_tile<DT, APPLY, MSR, PSR, EXACT, false, TJ>(c, L, hl, nest, false, sp, sl, false, TileSpan{}, red,
+                                                                 whole);
+            have0 = done && next.len > 0;
         }
     }
 }
