@@ -18,7 +18,7 @@
 //               its last lanes idle.
 //   KIND_QTEAM  multiples of 8 from 1032 to 4096: a workgroup per block, a
 //               quarter of it per wave, the absmax meeting in LDS.  In the
-//               generic list: blocks of 2048, one chunk per wave.
+//               generic list: blocks of up to 2048, one chunk per wave.
 //
 // Partial blocks (a leaf's last) take the same units, the lanes past the
 // leaf's end masked.  The weight-decay mode and eps_root are resolved at run
@@ -27,8 +27,8 @@
 // registers and branches).
 //
 // Bound: HBM, with the latency of a wave's chunk next.  One GPU, a 202 M
-// parameter bf16 layer (2.04 GB) in blocks of 256, nearest rounding: 437 us,
-// 4.66 TB/s, 57 VALU instructions per element (the 2048-element kernel: 43;
+// parameter bf16 layer (2.04 GB) in blocks of 256, nearest rounding: 435 us,
+// 4.7 TB/s, 58 VALU instructions per element (the 2048-element kernel: 43;
 // codes are scaled per element instead of through a per-block table, and the
 // reduction and reciprocals come per chunk).  What led there: 6.63 ms with a
 // workgroup per block, element accesses and two passes; 528 us with spans of
