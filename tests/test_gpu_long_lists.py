@@ -65,34 +65,35 @@ def _blocks():
     return 16 * torch.cuda.get_device_properties(0).multi_processor_count + 5
 
 
-@pytest.fixture(autouse=True)
-def longer_tree(monkeypatch, request):
-    """Another leaf in every tree: around rf.adamw8 and rf.adamw8_step (zero
-    grads, not compared), or, for grouped trees, in the module's own list of
-    leaves (compared like the rest)."""
+def lengthen(monkeypatch, function, **options):
+    """Another leaf in every tree of the test `function`: around rf.adamw8
+    (called with `options` too) and rf.adamw8_step (zero grads, not compared),
+    and, for grouped trees, in their module's own list of leaves (compared
+    like the rest)."""
     import torch
 
     import rollfast_amd as rf
 
     shape = (_blocks(), 2048)
-    if request.function.__module__ == groups.__name__:
+    build, step = rf.adamw8, rf.adamw8_step
+    if function.__module__ == groups.__name__:
         leaves = groups.LEAVES + [(PAD, shape, "bf16", "base")]
         monkeypatch.setattr(groups, "LEAVES", leaves)
         monkeypatch.setattr(groups, "LABELS", {name: lab for name, _s, _d, lab in leaves})
+        monkeypatch.setattr(rf, "adamw8", lambda *args, **kwargs: build(*args, **options, **kwargs))
         return
 
     pad = torch.full(shape, 0.01, dtype=torch.bfloat16, device="cuda")
     zero = torch.zeros_like(pad)
-    build, step = rf.adamw8, rf.adamw8_step
 
     def adamw8(*args, **kwargs):
-        tx = build(*args, **kwargs)
+        tx = build(*args, **options, **kwargs)
         return tx._replace(init=lambda params: tx.init({**params, PAD: pad}))
 
     def adamw8_step(tx, params, grads, state, *args, random_bits=None, **kwargs):
         n = len(params)
         if random_bits is not None:
-            words = torch.zeros(pad.numel(), dtype=torch.int32, device="cuda").view(torch.uint32)
+            words = torch.zeros(pad.numel() + 4096, dtype=torch.int32, device="cuda").view(torch.uint32)
             random_bits = {**random_bits, n: (words, words, words)}
         params, state = step(tx, {**params, PAD: pad}, {**grads, PAD: zero}, state, *args, random_bits=random_bits,
                              **kwargs)
@@ -102,3 +103,8 @@ def longer_tree(monkeypatch, request):
 
     monkeypatch.setattr(rf, "adamw8", adamw8)
     monkeypatch.setattr(rf, "adamw8_step", adamw8_step)
+
+
+@pytest.fixture(autouse=True)
+def longer_tree(monkeypatch, request):
+    lengthen(monkeypatch, request.function)
